@@ -62,8 +62,9 @@ struct vct_blocked {
 
 // LDS-resident form of a stage 1 (built with the blocked form unless
 // VCT_SYSMAT_NO_TILE): the stage-1 runs of each LDS block sorted by length
-// (longest first) in slices of 64, whose entries are interleaved so that lane
-// l of a wave reads entry k of run l at slice_ptr + 64 k + l.
+// (longest first) in slices of 64, whose entries are interleaved in fours so
+// that lane l of a wave reads entries 4 q .. 4 q + 3 of run l at slice_ptr +
+// 256 q + 4 l: a 16-byte load of lengths and an 8-byte load of LDS indices.
 //   forward: a block is a 64x64 image tile; an entry holds its voxel's index
 //     inside the tile (ly * 64 + lx) and the length; padding entries are
 //     (kTilePadVoxel, 0.0f), which read zeroed LDS;
@@ -74,9 +75,10 @@ struct vct_blocked {
 //     (0, 0.0f).
 struct vct_tiled {
     int ntiles = 0, nslices = 0, kmax = 0, ntx = 0;
-    uint2* ell = nullptr;            // [sum slice_len * 64 + 64 * kTileUnroll]
+    float* ell_len = nullptr;        // [sum slice_len * 64 + 64 * 2 * kTileUnroll] lengths
+    uint16_t* ell_idx = nullptr;     // the same entries' LDS indices
     uint32_t* slice_ptr = nullptr;   // [nslices] first entry of the slice
-    uint32_t* slice_len = nullptr;   // [nslices] entries per lane (adjoint: a multiple of kTileUnroll)
+    uint32_t* slice_len = nullptr;   // [nslices] entries per lane, a multiple of kTileUnroll
     int32_t* slice_runs = nullptr;   // [nslices * 64] stage-1 row of each lane, -1: none
     int32_t* tile_slices = nullptr;  // [ntiles + 1]
     int32_t* xcd_tiles = nullptr;    // [8 * kmax] tiles of each XCD, -1: none
@@ -99,8 +101,8 @@ struct vct_sysmat {
     uint32_t* col_ptr = nullptr;  // [NN+1]
     uint2* csc = nullptr;         // [nseg] (ray, float bits of length)
     vct_blocked fwd, adj;         // blocked forms (rows1 == 0: not built)
-    vct_tiled tile;               // LDS-resident forward stage 1 (ell == nullptr: not built)
-    vct_tiled atile;              // LDS-resident adjoint stage 1 (ell == nullptr: not built)
+    vct_tiled tile;               // LDS-resident forward stage 1 (ell_len == nullptr: not built)
+    vct_tiled atile;              // LDS-resident adjoint stage 1 (ell_len == nullptr: not built)
 };
 
 namespace vct {
@@ -971,11 +973,15 @@ __global__ void k_zero_f32(float* p, int n)
 // ------------------------------------------- tile-resident forward stage 1
 
 constexpr int kTileThreads = 1024;  // one workgroup per CU (LDS)
-constexpr int kTileUnroll = 8;      // entries in flight per lane
-// Tile-local voxel code of padding entries: "row 64", the zeroed LDS slots
-// after the tile, so padding adds exact zeros whatever the tile holds (an inf
-// or NaN density included).
-constexpr uint32_t kTilePadVoxel = 64u * 64u;
+constexpr int kTileUnroll = 4;      // entries per register set; slices hold a multiple of it
+// Tile rows in LDS are 67 voxels apart: rows 64 apart would put a column into
+// one bank, and of the odd pitches 67 gives the lanes' voxels the fewest bank
+// conflicts (1.8 cycles per conflict-free cycle over the runs of a tile at
+// 512^2 and M = 6; 65: 2.0).  An entry holds the voxel's index ly * 67 + lx.
+constexpr int kTilePitch = 67;
+// LDS index of padding entries: the zeroed slot after the tile, so padding
+// adds exact zeros whatever the tile holds (an inf or NaN density included).
+constexpr uint32_t kTilePadVoxel = 64u * kTilePitch;
 
 // Adjoint blocks.  A block is one part of a 64x64 tile in one view block:
 // the build splits each (view block, tile) into 1, 2, 4, 8 or 16 parts on a
@@ -990,14 +996,48 @@ constexpr int kAdjCells = 16;           // 16x16 cells of a 64x64 tile
 static_assert(kAdjTile == 64, "adjoint LDS blocks split 64x64 tiles into 4x4 cells of 16x16");
 constexpr int kAdjPadSlot = 0;
 
-__global__ __launch_bounds__(256) void k_fill_pad(uint2* __restrict__ p, size_t n, uint32_t pad)
+__global__ __launch_bounds__(256) void k_fill_pad(float* __restrict__ len, uint16_t* __restrict__ idx, size_t n,
+                                                  uint32_t pad)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = make_uint2(pad, 0u);
+    if (i >= n) return;
+    len[i] = 0.f;
+    idx[i] = (uint16_t)pad;
 }
 
-// Build: per stage-1 run, sort key tile << 16 | (0xffff - length) (longest
-// first within a tile), and the first run of each tile (the runs are in tile
+// Writes the n entries of a run (index and length from entry(k)) from dst on,
+// four at a time (the lane's next four are 256 further); entries past n are
+// padding.
+template <class F>
+__device__ __forceinline__ void ell_write(float* __restrict__ ell_len, uint16_t* __restrict__ ell_idx, size_t dst,
+                                          uint32_t n, uint32_t pad, F entry)
+{
+    for (uint32_t k0 = 0; k0 < n; k0 += 4, dst += 256) {
+        float l[4];
+        uint32_t x[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            l[u] = 0.f;
+            x[u] = pad;
+            if (k0 + u < n) entry(k0 + u, x[u], l[u]);
+        }
+        *reinterpret_cast<float4*>(ell_len + dst) = make_float4(l[0], l[1], l[2], l[3]);
+        *reinterpret_cast<ushort4*>(ell_idx + dst) =
+            make_ushort4((uint16_t)x[0], (uint16_t)x[1], (uint16_t)x[2], (uint16_t)x[3]);
+    }
+}
+
+// Length of a run in whole register sets.  Sorting by it (stably) instead of
+// by the length itself keeps runs of neighbouring rays (or voxels) that differ
+// by a segment or two in neighbouring lanes, whose LDS reads then mostly fall
+// in different banks, and costs no padding beyond the slices' own.
+__device__ __forceinline__ uint32_t tile_bucket(uint32_t len)
+{
+    return (len + kTileUnroll - 1) / kTileUnroll * kTileUnroll;
+}
+
+// Build: per stage-1 run, sort key tile << 16 | (0xffff - tile_bucket(length))
+// (longest first within a tile), and the first run of each tile (the runs are in tile
 // order, so each tile has one first run; no counter is contended).
 __global__ __launch_bounds__(256) void k_tile_run_keys(const uint32_t* __restrict__ ptr1, const uint2* __restrict__ ent1,
                                                        uint32_t rows1, TileGrid tg, uint32_t* __restrict__ key,
@@ -1009,8 +1049,8 @@ __global__ __launch_bounds__(256) void k_tile_run_keys(const uint32_t* __restric
     const uint32_t len = ptr1[r + 1] - ptr1[r];
     const uint32_t t = tg.tile(ent1[ptr1[r]].x);
     const uint32_t tp = r ? tg.tile(ent1[ptr1[r - 1]].x) : 0xffffffffu;
-    if (len == 0u || len >= 0xffffu || (r && t < tp)) atomicOr(err, 1u);
-    key[r] = (t << 16) | (0xffffu - min(len, 0xfffeu));
+    if (len == 0u || len > 0xfffcu || (r && t < tp)) atomicOr(err, 1u);
+    key[r] = (t << 16) | (0xffffu - tile_bucket(min(len, 0xfffcu)));
     val[r] = r;
     if (t != tp) tile_first[t] = r;
 }
@@ -1027,7 +1067,7 @@ __global__ void k_first_to_count(uint32_t* __restrict__ c, int ntiles, uint32_t 
     }
 }
 
-// Build: entries per lane of each slice = the length of its first (longest) run.
+// Build: entries per lane of each slice = the bucket of its first (longest) run.
 __global__ __launch_bounds__(256) void k_tile_slice_len(const uint32_t* __restrict__ ptr1, const uint32_t* __restrict__ order,
                                                         const int32_t* __restrict__ slice_tile,
                                                         const uint32_t* __restrict__ tile_begin,
@@ -1038,7 +1078,7 @@ __global__ __launch_bounds__(256) void k_tile_slice_len(const uint32_t* __restri
     if (sl >= nslices) return;
     const int t = slice_tile[sl];
     const uint32_t r = order[tile_begin[t] + (uint32_t)(sl - tile_slices[t]) * 64u];
-    slice_len[sl] = ptr1[r + 1] - ptr1[r];
+    slice_len[sl] = tile_bucket(ptr1[r + 1] - ptr1[r]);
 }
 
 // Build: the interleaved entries with tile-local voxel indices, one thread
@@ -1048,7 +1088,8 @@ __global__ __launch_bounds__(256) void k_tile_fill(const uint32_t* __restrict__ 
                                                    uint32_t rows1, const uint32_t* __restrict__ tile_begin,
                                                    const int32_t* __restrict__ tile_slices,
                                                    const uint32_t* __restrict__ slice_ptr, TileGrid tg,
-                                                   uint2* __restrict__ ell, int32_t* __restrict__ slice_runs,
+                                                   float* __restrict__ ell_len, uint16_t* __restrict__ ell_idx,
+                                                   int32_t* __restrict__ slice_runs,
                                                    uint32_t* __restrict__ err)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1058,14 +1099,16 @@ __global__ __launch_bounds__(256) void k_tile_fill(const uint32_t* __restrict__ 
     const uint32_t sl = (uint32_t)tile_slices[t] + p / 64u, lane = p % 64u;
     slice_runs[sl * 64u + lane] = (int32_t)r;
     const uint32_t tx0 = (t % (uint32_t)tg.ntx) * 64u, ty0 = (t / (uint32_t)tg.ntx) * 64u;
-    uint2* dst = ell + slice_ptr[sl] + lane;
-    for (uint32_t j = ptr1[r], k = 0; j < ptr1[r + 1]; j++, k++) {
-        const uint2 e = ent1[j];
+    const size_t dst = (size_t)slice_ptr[sl] + 4u * lane;
+    const uint32_t j0 = ptr1[r];
+    ell_write(ell_len, ell_idx, dst, ptr1[r + 1] - j0, kTilePadVoxel, [&](uint32_t k, uint32_t& x, float& l) {
+        const uint2 e = ent1[j0 + k];
         const uint32_t iy = e.x / (uint32_t)tg.N, ix = e.x - iy * (uint32_t)tg.N;
         const uint32_t ly = iy - ty0, lx = ix - tx0;  // wraps above 63 if outside the tile
         if (ly > 63u || lx > 63u) atomicOr(err, 2u);
-        dst[(size_t)k * 64u] = make_uint2((ly & 63u) * 64u + (lx & 63u), e.y);
-    }
+        x = (ly & 63u) * kTilePitch + (lx & 63u);
+        l = __uint_as_float(e.y);
+    });
 }
 
 // Adjoint build: the first stage-1 run of each blocked-form key (view block
@@ -1140,11 +1183,11 @@ __global__ __launch_bounds__(256) void k_atile_run_keys(const uint32_t* __restri
     if (r >= rows1) return;
     const uint32_t len = ptr1[r + 1] - ptr1[r];
     const uint32_t bt = cell_block[(size_t)key1[r] * kAdjCells + adj_cell(row1[r], N)];
-    if (len == 0u || len >= 0xffffu || bt >= nblocks) {
+    if (len == 0u || len > 0xfffcu || bt >= nblocks) {
         atomicOr(err, 1u);
         key[r] = 0u;
     } else {
-        key[r] = (bt << 16) | (0xffffu - len);
+        key[r] = (bt << 16) | (0xffffu - tile_bucket(len));
         atomicAdd(cnt + bt, 1u);
     }
     val[r] = r;
@@ -1161,7 +1204,8 @@ __global__ __launch_bounds__(256) void k_atile_fill(const uint32_t* __restrict__
                                                     const int32_t* __restrict__ slot_off,
                                                     const int32_t* __restrict__ slot_clo,
                                                     const int32_t* __restrict__ blk_v0, int W,
-                                                    uint2* __restrict__ ell, int32_t* __restrict__ slice_runs,
+                                                    float* __restrict__ ell_len, uint16_t* __restrict__ ell_idx,
+                                                    int32_t* __restrict__ slice_runs,
                                                     uint32_t* __restrict__ err)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1173,9 +1217,10 @@ __global__ __launch_bounds__(256) void k_atile_fill(const uint32_t* __restrict__
     const uint32_t v0 = (uint32_t)blk_v0[K];
     const int32_t* off = slot_off + (size_t)K * (kAdjViews + 1);
     const int32_t* clo = slot_clo + (size_t)K * kAdjViews;
-    uint2* dst = ell + slice_ptr[sl] + lane;
-    for (uint32_t j = ptr1[r], k = 0; j < ptr1[r + 1]; j++, k++) {
-        const uint2 e = ent1[j];
+    const size_t dst = (size_t)slice_ptr[sl] + 4u * lane;
+    const uint32_t j0 = ptr1[r];
+    ell_write(ell_len, ell_idx, dst, ptr1[r + 1] - j0, (uint32_t)kAdjPadSlot, [&](uint32_t k, uint32_t& x, float& l) {
+        const uint2 e = ent1[j0 + k];
         const uint32_t v = e.x / (uint32_t)W, c = e.x - v * (uint32_t)W, jv = v - v0;
         uint32_t slot = (uint32_t)kAdjPadSlot;
         if (jv < (uint32_t)kAdjViews) {
@@ -1185,20 +1230,23 @@ __global__ __launch_bounds__(256) void k_atile_fill(const uint32_t* __restrict__
         } else {
             atomicOr(err, 4u);
         }
-        dst[(size_t)k * 64u] = make_uint2(slot, e.y);
-    }
+        x = slot;
+        l = __uint_as_float(e.y);
+    });
 }
 
 struct TileArgs {
     const float* in;             // densities (forward) or ray weights (adjoint): rows of 8*B floats
     float* out;                  // stage-1 partial sums: rows of 8*B floats
-    const uint2* ell;
+    const float* ell_len;
+    const uint16_t* ell_idx;
     const uint32_t* slice_ptr;
     const uint32_t* slice_len;
     const int32_t* slice_runs;
     const int32_t* tile_slices;
     const int32_t* xcd_tiles;
     int kmax, ntx, N, B;
+    int parts;                   // workgroups that share the slices of one (block, phantom)
     const int32_t* slot_off;     // adjoint: ray tables of the blocks
     const int32_t* slot_clo;
     const int32_t* blk_v0;
@@ -1238,6 +1286,11 @@ __global__ __launch_bounds__(256) void k_weights_pm(const float* __restrict__ in
 // Each lane then sums one run of a slice in FP64, 8 entries in flight, and
 // writes its partial sums as stage-1 row run, phantom b.  The sums are those
 // of k_gather over the same runs, term for term in the same order.
+// Bound by what passes between L2 and the CU: at 16 phantoms of 512^2, M = 6,
+// a copy without the LDS reads or without the sums takes the same 3.8 ms, one
+// without the entry loads 2.3 ms, one without the stores 3.0 (forward).  So
+// entries are 6 bytes (16-bit LDS index, float length) in two wide loads per
+// four: forward 3.81 -> 3.23 ms, adjoint 3.85 -> 3.75 against 8-byte entries.
 // Several groups (one per geometry) in one launch: workgroup l belongs to the
 // group gi with pref[gi] <= l < pref[gi + 1] (a scalar search).  Each group's
 // range is a multiple of 8 workgroups, so l - pref[gi] keeps l's XCD.
@@ -1254,14 +1307,13 @@ __global__ __launch_bounds__(ADJ ? kAtileThreads : kTileThreads) void k_gather_t
     while (gi + 1 < ga.n && (int)blockIdx.x >= ga.pref[gi + 1]) gi++;
     const TileArgs& a = ga.a[gi];
     constexpr int MP = (M + 1) & ~1;  // floats per voxel or ray in LDS
-    constexpr int ROW = 64 * MP + 2;  // floats per tile row (forward)
     constexpr int U = kTileUnroll;
-    constexpr int LDSF = ADJ ? kAdjSlotCap * MP : 64 * ROW + 8;
-    constexpr uint32_t PAD = ADJ ? (uint32_t)kAdjPadSlot : kTilePadVoxel;
+    constexpr int LDSF = ADJ ? kAdjSlotCap * MP : (64 * kTilePitch + 1) * MP;
     __shared__ float lds[LDSF];
     __shared__ int32_t tab[2 * kAdjViews + 2];  // adjoint: slot_off, slot_clo, first view of the block
     const int g = (int)blockIdx.x - ga.pref[gi], xcd = g % kXcds, slot = g / kXcds;
-    const int k = slot / a.B, b = slot % a.B;
+    // the phantoms of one part of a block side by side: they read the same entries
+    const int per = a.B * a.parts, k = slot / per, part = slot % per / a.B, b = slot % a.B;
     if (k >= a.kmax) return;  // the whole workgroup
     const int t = a.xcd_tiles[xcd * a.kmax + k];
     if (t < 0) return;
@@ -1309,59 +1361,93 @@ __global__ __launch_bounds__(ADJ ? kAtileThreads : kTileThreads) void k_gather_t
         }
     } else {
         const int tx0 = (t % a.ntx) * 64, ty0 = (t / a.ntx) * 64;
-        if (threadIdx.x < 8) lds[64 * ROW + threadIdx.x] = 0.f;
+        if (threadIdx.x < MP) lds[kTilePadVoxel * MP + threadIdx.x] = 0.f;
         for (int i = threadIdx.x; i < 64 * 64; i += blockDim.x) {
             const int ly = i >> 6, lx = i & 63, gy = ty0 + ly, gx = tx0 + lx;
             float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (gy < a.N && gx < a.N) load_slot<M>(a.in, (size_t)gy * a.N + gx, a.B, b, v);
-            float2* d = reinterpret_cast<float2*>(lds + ly * ROW + lx * MP);
+            float2* d = reinterpret_cast<float2*>(lds + (ly * kTilePitch + lx) * MP);
 #pragma unroll
             for (int q = 0; q < MP / 2; q++) d[q] = make_float2(v[2 * q], v[2 * q + 1]);
         }
     }
     __syncthreads();
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-    for (int sl = a.tile_slices[t] + w; sl < a.tile_slices[t + 1]; sl += nw) {
-        const int len = (int)a.slice_len[sl];
-        const uint2* e = a.ell + a.slice_ptr[sl] + lane;
+    // the wave's slice, its length and its entries' base are scalars, so the
+    // loop control runs on the scalar unit and an entry load is one
+    // instruction (scalar base, lane offset)
+    const int lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int last = a.tile_slices[t + 1], step = nw * a.parts;
+    int sl = a.tile_slices[t] + part * nw + w, nsl = sl;
+    int len = sl < last ? (int)a.slice_len[sl] : 0;
+    uint32_t ptr = sl < last ? a.slice_ptr[sl] : 0u;
+    for (; sl < last; sl = nsl) {
+        len = __builtin_amdgcn_readfirstlane(len);
+        const uint32_t e0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ptr);
+        const float* elen = a.ell_len + e0;
+        const uint16_t* eidx = a.ell_idx + e0;
         double acc[MP];
 #pragma unroll
         for (int m = 0; m < MP; m++) acc[m] = 0.0;
-        uint2 q[U], nq[U];
-        // padding entries (runs shorter than the slice, and in the forward
-        // past len) are (PAD, 0.0f): zero LDS data times zero length.  An
-        // adjoint len is a multiple of U, and the last prefetch reads the
-        // next slice or the slack after the last one.
-#pragma unroll
-        for (int u = 0; u < U; u++) q[u] = ADJ || u < len ? e[u * 64] : make_uint2(PAD, 0u);
-        for (int j = 0; j < len; j += U) {
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                nq[u] = ADJ || j + U + u < len ? e[(j + U + u) * 64] : make_uint2(PAD, 0u);
+        struct Set {
+            float4 len;
+            ushort4 idx;
+        };
+        static_assert(U == 4, "a register set holds the four entries of one load");
+        auto fetch = [&](Set& q, int j) {
+            q.len = reinterpret_cast<const float4*>(elen + (size_t)(uint32_t)j * 64u)[(uint32_t)lane];
+            q.idx = reinterpret_cast<const ushort4*>(eidx + (size_t)(uint32_t)j * 64u)[(uint32_t)lane];
+            // (the loads are issued here: without this the compiler sinks them
+            // past the loop's exits to their first use)
+            asm volatile("" ::: "memory");
+        };
+        auto sum = [&](const Set& q) {
+            const float ln[U] = {q.len.x, q.len.y, q.len.z, q.len.w};
+            const uint32_t ix[U] = {q.idx.x, q.idx.y, q.idx.z, q.idx.w};
             float2 f[U][MP / 2];
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                // 24-bit multiplies (full rate; v_mul_lo_u32 is quarter rate):
-                // slots and tile rows are far below 2^24
-                const float* base = ADJ ? lds + __umul24(q[u].x, (unsigned)MP)
-                                        : lds + __umul24(q[u].x >> 6, (unsigned)ROW) + (q[u].x & 63) * MP;
-                const float2* p = reinterpret_cast<const float2*>(base);
+                // (24-bit multiply: full rate, v_mul_lo_u32 is quarter rate)
+                const float2* p = reinterpret_cast<const float2*>(lds + __umul24(ix[u], (unsigned)MP));
 #pragma unroll
                 for (int h = 0; h < MP / 2; h++) f[u][h] = p[h];
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const double v = __uint_as_float(q[u].y);
+                const double v = ln[u];
 #pragma unroll
                 for (int h = 0; h < MP / 2; h++) {
                     acc[2 * h] = __builtin_fma((double)f[u][h].x, v, acc[2 * h]);
                     acc[2 * h + 1] = __builtin_fma((double)f[u][h].y, v, acc[2 * h + 1]);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < U; u++) q[u] = nq[u];
-        }
+        };
+        // Three register sets of U entries in turn, two of them in flight
+        // while the third is summed (no copies between the sets).  len is a
+        // multiple of U; padding entries (runs shorter than the slice) read a
+        // zero slot and have length 0.  The last fetches read up to 2 U
+        // entries past the slice: the next slice or the slack after the last.
+        Set q0, q1, q2;
+        fetch(q0, 0);
+        fetch(q1, U);
         const int run = a.slice_runs[sl * 64 + lane];
+        const int this_len = len;
+        nsl = sl + step;
+        if (nsl < last) {
+            len = (int)a.slice_len[nsl];
+            ptr = a.slice_ptr[nsl];
+        }
+        for (int j = 0;;) {
+            fetch(q2, j + 2 * U);
+            sum(q0);
+            if ((j += U) >= this_len) break;
+            fetch(q0, j + 2 * U);
+            sum(q1);
+            if ((j += U) >= this_len) break;
+            fetch(q1, j + 2 * U);
+            sum(q2);
+            if ((j += U) >= this_len) break;
+        }
         if (run >= 0) {
             float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1503,7 +1589,7 @@ static vct_status build_blocked(const uint2* ent, const uint32_t* row_of, uint32
 
 static void free_tiled(vct_tiled& t)
 {
-    void* bufs[] = {t.ell,         t.slice_ptr, t.slice_len, t.slice_runs, t.tile_slices,
+    void* bufs[] = {t.ell_len,     t.ell_idx, t.slice_ptr, t.slice_len, t.slice_runs, t.tile_slices,
                     t.xcd_tiles,   t.slot_off,  t.slot_clo,  t.blk_v0};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -1772,10 +1858,6 @@ static vct_status build_tiled(const vct_blocked& f, const TileGrid& tg, vct_tile
     std::vector<uint64_t> work(nblocks, 0);
     if (ok && st == VCT_OK) {
         for (int sl = 0; sl < nslices; sl++) {
-            // adjoint slices hold a multiple of kTileUnroll entries per lane,
-            // so the kernel reads them without bounds tests (the forward's
-            // short runs near tile edges would pay more padding than it saves)
-            if (adj) slen[sl] = (slen[sl] + kTileUnroll - 1) / kTileUnroll * kTileUnroll;
             sptr[sl] = (uint32_t)total;
             total += 64ull * slen[sl];
             work[stile[sl]] += 64ull * slen[sl];
@@ -1821,23 +1903,24 @@ static vct_status build_tiled(const vct_blocked& f, const TileGrid& tg, vct_tile
         t.kmax = kmax;
         t.n_ell = (size_t)total;
         hip(hipMalloc(&t.xcd_tiles, 4 * xt.size()), "hipMalloc xcd tiles");
-        const size_t n_fill = (size_t)total + 64 * kTileUnroll;  // slack for the adjoint's last prefetch
-        hip(hipMalloc(&t.ell, 8 * n_fill), "hipMalloc tile entries");
+        const size_t n_fill = (size_t)total + 64 * 2 * kTileUnroll;  // slack for the last slice's prefetches
+        hip(hipMalloc(&t.ell_len, 4 * n_fill), "hipMalloc tile entries");
+        hip(hipMalloc(&t.ell_idx, 2 * n_fill), "hipMalloc tile entries");
         if (st == VCT_OK) {
             hip(hipMemcpyAsync(t.xcd_tiles, xt.data(), 4 * xt.size(), hipMemcpyHostToDevice, s), "copy");
             hip(hipMemcpyAsync(t.slice_ptr, sptr.data(), 4 * (size_t)nslices, hipMemcpyHostToDevice, s), "copy");
-            hip(hipMemcpyAsync(t.slice_len, slen.data(), 4 * (size_t)nslices, hipMemcpyHostToDevice, s), "copy");
-            hipLaunchKernelGGL(k_fill_pad, dim3((unsigned)((n_fill + 255) / 256)), blk, 0, s, t.ell, n_fill,
+            hipLaunchKernelGGL(k_fill_pad, dim3((unsigned)((n_fill + 255) / 256)), blk, 0, s, t.ell_len,
+                               t.ell_idx, n_fill,
                                adj ? (uint32_t)kAdjPadSlot : kTilePadVoxel);
             hip(hipMemsetAsync(t.slice_runs, 0xff, 4 * 64 * (size_t)nslices, s), "memset");
             hipLaunchKernelGGL(k_zero_f32, dim3(1), blk, 0, s, (float*)err, 1);
             if (adj)
                 hipLaunchKernelGGL(k_atile_fill, gr, blk, 0, s, f.ptr1, f.ent1, key_s, order, R, tile_begin,
-                                   t.tile_slices, t.slice_ptr, t.slot_off, t.slot_clo, t.blk_v0, adj->W, t.ell,
-                                   t.slice_runs, err);
+                                   t.tile_slices, t.slice_ptr, t.slot_off, t.slot_clo, t.blk_v0, adj->W, t.ell_len,
+                                   t.ell_idx,                                   t.slice_runs, err);
             else
                 hipLaunchKernelGGL(k_tile_fill, gr, blk, 0, s, f.ptr1, f.ent1, key_s, order, R, tile_begin,
-                                   t.tile_slices, t.slice_ptr, tg, t.ell, t.slice_runs, err);
+                                   t.tile_slices, t.slice_ptr, tg, t.ell_len, t.ell_idx, t.slice_runs, err);
             hip(hipGetLastError(), "tile fill");
             hip(hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, s), "copy");
             hip(hipStreamSynchronize(s), "sync");
@@ -1847,7 +1930,7 @@ static vct_status build_tiled(const vct_blocked& f, const TileGrid& tg, vct_tile
     void* bufs[] = {key, key_s, val, order, cnt, err, tile_begin, slice_tile, cell_block, tmp};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (st != VCT_OK || !ok || !t.ell) free_tiled(t);
+    if (st != VCT_OK || !ok || !t.ell_idx) free_tiled(t);
     return st;
 }
 
@@ -2036,8 +2119,8 @@ size_t vct_sysmat_bytes(const vct_sysmat* m)
             b += sizeof(uint2) * (size_t)m->nseg + sizeof(uint32_t) * ((size_t)fs[k]->rows1 + 1) +
                  sizeof(uint32_t) * ((size_t)rows[k] + 1) + sizeof(uint2) * ((size_t)fs[k]->rows1 + 1);
     for (const vct_tiled* t : {&m->tile, &m->atile})
-        if (t->ell)
-            b += sizeof(uint2) * t->n_ell + sizeof(uint32_t) * 66 * (size_t)t->nslices +
+        if (t->ell_len)
+            b += (sizeof(float) + sizeof(uint16_t)) * t->n_ell + sizeof(uint32_t) * 66 * (size_t)t->nslices +
                  sizeof(int32_t) * ((size_t)t->ntiles + 1 + (size_t)kXcds * t->kmax) +
                  (t->slot_off ? sizeof(int32_t) * (2 * kAdjViews + 1) * (size_t)t->ntiles : 0);
     return b;
@@ -2055,7 +2138,7 @@ static size_t pm_offset(const vct_sysmat* m, int B)
 size_t vct_sysmat_workspace(const vct_sysmat* m, int n_phantoms)
 {
     if (!m || n_phantoms < 1) return 0;
-    const size_t pm = m->atile.ell ? (size_t)m->nrays * n_phantoms * 8 * sizeof(float) : 0;
+    const size_t pm = m->atile.ell_len ? (size_t)m->nrays * n_phantoms * 8 * sizeof(float) : 0;
     return pm_offset(m, n_phantoms) + pm;
 }
 
@@ -2102,12 +2185,23 @@ static vct_status run_gather(GatherArgs& a, int items, int M, int lanes, int blo
 static const vct_tiled* lds_form(const vct_sysmat* m, bool adjoint)
 {
     const vct_tiled& t = adjoint ? m->atile : m->tile;
-    if (!t.ell || (adjoint && t.slots_max > kAdjSlotCap)) return nullptr;
+    if (!t.ell_len || (adjoint && t.slots_max > kAdjSlotCap)) return nullptr;
     return &t;
 }
 
+// Workgroups per (block, phantom): enough for about eight workgroups per CU
+// over the launch (a few large blocks would leave CUs idle: 3 phantoms of
+// 200^2 are 48 workgroups, a solver step 2.03 ms, 1.10 with 16 parts), as long
+// as each keeps 64 slices to sum against its fill of LDS.
+static int tile_parts(const vct_tiled& t, int B)
+{
+    const long long wgs = std::max(1LL, (long long)t.ntiles * B);
+    const long long want = (2048 + wgs - 1) / wgs, most = std::max(1LL, (long long)t.nslices / t.ntiles / 64);
+    return (int)std::max(1LL, std::min({want, most, 16LL}));
+}
+
 // Stage 1 of the groups over their LDS-resident forms in one launch: per
-// group B workgroups per block, kmax blocks per XCD.
+// group B * parts workgroups per block, kmax blocks per XCD.
 static vct_status run_gather_tile(const vct_batch_group* groups, const int* idx, const vct_tiled* const* forms, int n,
                                   bool adjoint, int M, hipStream_t s)
 {
@@ -2132,11 +2226,12 @@ static vct_status run_gather_tile(const vct_batch_group* groups, const int* idx,
             VCT_PM_M(5) VCT_PM_M(6) VCT_PM_M(7) VCT_PM_M(8)
 #undef VCT_PM_M
         }
-        tg.a[q] = TileArgs{G.d_in, G.d_work, t.ell, t.slice_ptr, t.slice_len, t.slice_runs, t.tile_slices,
-                           t.xcd_tiles, t.kmax, t.ntx, G.sysmat->plan->g.recon_size, G.n_phantoms, t.slot_off,
+        const int parts = tile_parts(t, G.n_phantoms);
+        tg.a[q] = TileArgs{G.d_in, G.d_work, t.ell_len, t.ell_idx, t.slice_ptr, t.slice_len, t.slice_runs, t.tile_slices,
+                           t.xcd_tiles, t.kmax, t.ntx, G.sysmat->plan->g.recon_size, G.n_phantoms, parts, t.slot_off,
                            t.slot_clo, t.blk_v0, G.sysmat->plan->g.n_channels, pm, G.sysmat->nrays};
         tg.pref[q] = (int)total;
-        total += (long long)kXcds * t.kmax * G.n_phantoms;  // a multiple of kXcds
+        total += (long long)kXcds * t.kmax * G.n_phantoms * parts;  // a multiple of kXcds
         if (total > INT_MAX) return set_error(VCT_ERR_ARG, "stage-1 launch too large");
     }
     tg.pref[n] = (int)total;
