@@ -127,6 +127,7 @@ struct BpGroups {
     int n;
 };
 
+constexpr int kNpfPoly = 13;
 struct LengthprojArgs {
     const float* proj;    // [count][W] sinogram window
     const double* cosT;   // [V]
@@ -138,6 +139,7 @@ struct LengthprojArgs {
     int count;            // window rows (V/2*2)
     double pix, rz, sid, det_src_iso, det_radius, iso_det, iso_channel;
     double delta;         // channel pitch in radians, max_alpha / ((W-1)/2)
+    double poly[kNpfPoly];  // channels per unit tan: the fan form's polynomial
 };
 
 }  // namespace vct
