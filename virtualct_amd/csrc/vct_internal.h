@@ -105,6 +105,7 @@ struct FilterGemmArgs {
     int edge_lo, edge_hi; // output columns m <= edge_lo or m >= edge_hi are renormalised rows
 };
 
+constexpr int kBpPoly = 9;
 struct BackprojArgs {
     const float* fltd;    // [S][V][W]
     const double* cosT;   // [V]
@@ -114,6 +115,7 @@ struct BackprojArgs {
     int exact;            // 1: views in the reference's order per pixel, no 4-fold sharing
     int max_k;            // most sinograms per lane of the multi-sinogram kernel (0: kBpSinos)
     double pix, sid, dbeta_ch, inv_dbeta_ch, dbeta_view, xfactor, center, mask_r2, mask_r;
+    double poly[kBpPoly] = {};  // channels per unit tan(gamma): the float-weight form's polynomial
 };
 
 // Backprojections of up to kMaxBpGroups geometries in one launch
