@@ -142,8 +142,9 @@ vct_status vct_plan_destroy(vct_plan* plan);
  * test can fire use one ray per march.
  * Launch shapes (results do not depend on them, beyond the order of float
  * adds where noted; an autotuner times them per shape):
- * VCT_OPT_TRACE_BLOCK = 6: lanes per workgroup of the tracer, 64, 128 or 256
- * (0: 64).
+ * VCT_OPT_TRACE_BLOCK = 6: lanes per workgroup, 64, 128 or 256 (0: 64), of
+ * the tracers that march step by step (the exact option, the r >= rmax test,
+ * grids whose plane middles fall on grid lines); the others use 512.
  * VCT_OPT_BP_SINOS_PER_LANE = 7: most sinograms one lane backprojects in a
  * multi-sinogram call, 2..16 (0: 16); images are bit-identical for every value.
  * VCT_OPT_ADJOINT_VIEWS = 8: views per workgroup of the adjoint, 1..256 (0: a
@@ -194,11 +195,12 @@ vct_status vct_pack_densities_f32(vct_plan* plan, const float* d_dens, int M,
  * ray's segments of rho_m * length, g/cm^2, divided by xfactor).  Each ray
  * is traced once, independent of the spectrum.  d_counts (optional, int32
  * [V][W]) receives the reference's per-ray segment counter
- * (reprojection_sum, :195/:280).  With orbits (VCT_OPT_TRACE_ORBIT), the
- * call first writes d_packed and its transpose, each padded by two voxels,
- * into a work buffer that the plan allocates with itself (64*(N+4)^2 bytes
- * when N and V are even), so that the gathers of rays along x read rows
- * too. */
+ * (reprojection_sum, :195/:280).  The call first writes d_packed and its
+ * transpose, each padded by two voxels, into a work buffer that the plan
+ * allocates with itself (64*(N+4)^2 bytes and a bit per ray), so that the
+ * gathers of rays along x read rows too; calls on one plan must not overlap.
+ * The exact option and geometries where the reference's r >= rmax test can
+ * fire read d_packed itself. */
 vct_status vct_trace_paths(vct_plan* plan, const void* d_packed, int dens_type, int M,
                            float* d_L, int32_t* d_counts, void* stream);
 

@@ -340,3 +340,40 @@ def test_orbit_trace_equals_single_ray_march(gpu, golden, N, pix, V):
             # float32 outputs of FP64 sums that differ in the last bits: at
             # most one float ulp apart (1.2e-7 of the largest value)
             assert rel_max(L, L1) < 2.5e-7, (orbit, name)
+
+
+@pytest.mark.parametrize("N,fov,V,W,M,f32", [
+    (6, 2.0, 4, 22, 1, False), (7, 2.0, 5, 23, 3, True), (64, 50.0, 80, 609, 6, False), (64, 51.2, 80, 609, 6, False),
+    (128, 51.2, 48, 609, 6, True), (130, 50.0, 12, 333, 8, True), (130, 50.0, 14, 64, 8, False),
+    (301, 50.0, 9, 65, 2, True), (256, 50.0, 20, 609, 5, False), (96, 30.0, 36, 80, 7, False), (33, 20.0, 6, 47, 4, True)])
+def test_segment_tracer_equals_exact_march(gpu, N, fov, V, W, M, f32):
+    """The segment-by-segment tracer (orbits of 4, 2 and 1 rays, partial tiles
+    of 16 channels x 4 views, an odd count's last view, odd N; at 128 voxels
+    on 51.2 cm the step-by-step form that such grids keep) against the
+    exact-division march of every ray: the same segment counters, and path
+    integrals within two float roundings, since both sum the same segments in
+    FP64 with lengths equal to ~1e-11.  Some densities are negative and NaN,
+    which contribute nothing."""
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    geom = default_geometry(recon_size=N, pixel_cm=fov / N, n_views=V, n_channels=W, iso_channel=W / 2.0 + 0.13)
+    rng = np.random.default_rng(N + V)
+    if f32:
+        d = rng.uniform(0.0, 2.0, (M, N, N)).astype(np.float32)
+        d[:, 0, 0] = -1.0
+        d[:, N // 2, 1] = np.nan
+    else:
+        d = rng.integers(0, 2000, (M, N, N)).astype(np.int16)
+        d[:, 0, 0] = -5
+    out = []
+    for exact in (0, 1):
+        plan = ops.Plan(geom)
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        pk, dt = ops.pack_densities(plan, _t(d, gpu))
+        L, cnt = ops.trace_paths(plan, pk, dt, M, counts=True)
+        out.append((L.cpu().numpy(), cnt.cpu().numpy()))
+        plan.close()
+    (L, c), (Le, ce) = out
+    np.testing.assert_array_equal(c, ce)
+    assert np.isfinite(L).all() and not np.any(L[..., M:])
+    assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9)

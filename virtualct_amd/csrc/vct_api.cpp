@@ -107,6 +107,7 @@ TraceArgs make_trace_args(const vct_plan* p)
     a.block = p->trace_block > 0 ? p->trace_block : 64;
     a.adj_views = p->adj_views;
     a.dens_t = p->d_dens_t;
+    a.redo = p->d_redo;
     // orbits of the half or quarter turn: every view traced (V even), a grid
     // centred on a voxel corner (N even), the guarded march (no exact option,
     // no r >= rmax test)
@@ -386,13 +387,15 @@ vct_status vct_plan_create(vct_ctx* ctx, const vct_geometry* g, vct_plan** out)
     if (st == VCT_OK) st = plan_upload(coeff.data(), W * sizeof(double), (void**)&p->d_coeff);
     // the orbit tracer's work copies (any dens type), allocated with the
     // plan so that no trace call allocates
-    if (st == VCT_OK && g->recon_size % 2 == 0 && V % 2 == 0) {
-        // two padded copies of (N + 4)^2 voxels of up to 32 bytes
-        const size_t np = (size_t)g->recon_size + 4;
-        const size_t bytes = 2 * np * np * 32;
+    if (st == VCT_OK) {
+        // two padded copies of (N + 4)^2 voxels of up to 32 bytes, the redo bits
+        const size_t np = (size_t)g->recon_size + 4, copies = 2 * np * np * 32;
+        const size_t bytes = copies + trace_redo_words(V, W) * 8;
         if (hipMalloc(&p->d_dens_t, bytes) != hipSuccess) {
             (void)hipGetLastError();
             st = set_error(VCT_ERR_NOMEM, "plan work copy of %zu bytes", bytes);
+        } else {
+            p->d_redo = reinterpret_cast<unsigned long long*>(static_cast<char*>(p->d_dens_t) + copies);
         }
     }
     if (st != VCT_OK) {

@@ -42,7 +42,8 @@ struct TraceArgs {
     const double* px0;    // [W] detector point before rotation (x)
     const double* py0;    // [W] detector point before rotation (y)
     const void* dens;     // packed [N][N][8] (u16 or f32)
-    void* dens_t;         // orbit tracer: work copies of dens, [y][x] and [x][y], padded to N + 4
+    void* dens_t;         // tracer: work copies of dens, [y][x] and [x][y], padded to N + 4
+    unsigned long long* redo;  // tracer: orbits left to the ray by ray march, a bit each
     float* L;             // [V][W][8] path integrals (forward)
     int32_t* counts;      // [V][W] optional segment counter
     const float* wts;     // [V][W][8] adjoint weights (adjoint)
@@ -177,7 +178,8 @@ struct vct_plan {
     double* d_coeff = nullptr;
     float* d_bpk[3] = {nullptr, nullptr, nullptr};   // packed filter matrix per type
     float* d_toep[3] = {nullptr, nullptr, nullptr};  // Toeplitz generator per type
-    void* d_dens_t = nullptr;  // the orbit tracer's density work copies (N, V even)
+    void* d_dens_t = nullptr;  // the tracer's density work copies, then its redo bits
+    unsigned long long* d_redo = nullptr;  // inside d_dens_t
     int exact_trace = 0;  // VCT_OPT_EXACT_TRACE
     int max_steps = 0;    // VCT_OPT_MAX_STEPS (0: the automatic bound)
     int exact_bp = 0;     // VCT_OPT_EXACT_BACKPROJECT
@@ -190,6 +192,7 @@ struct vct_plan {
 namespace vct {
 // kernels launchers (implemented in the .hip files)
 vct_status launch_trace(const TraceArgs& a, int dens_type, int M, bool adjoint, hipStream_t s);
+size_t trace_redo_words(int V, int W);  // 64-bit words of TraceArgs::redo
 vct_status launch_spectral(const SpectralArgs& a, hipStream_t s);
 vct_status launch_stats_init(uint32_t* stats, int S, hipStream_t s);
 vct_status launch_detector(const DetectorArgs& a, hipStream_t s);

@@ -17,9 +17,13 @@
 //                max/min used by the normalisation and the noise clamp.
 //   k_detector   max-normalisation + Gaussian noise (Philox4x32-10 +
 //                Box-Muller) + the reference's clamps.
-//   k_trace_fwd_rot  the quarter- (or half-) turn orbit form: one march
-//                for the rays of views v, v + V/4, v + V/2, v + 3V/4, split
-//                over eight lanes by step windows.
+//   k_trace_seg  the same path integrals with one segment per loop iteration,
+//                one march for the rays of views v, v + V/4, v + V/2,
+//                v + 3V/4 (or v, v + V/2, or one ray); k_trace_redo marches
+//                what it leaves undecided.
+//   k_trace_fwd_rot  the quarter- (or half-) turn orbit form of k_trace_fwd,
+//                split over eight lanes by step windows, for the grids that
+//                k_trace_seg does not take (seg_grid).
 //   k_trace_adj_tile  the adjoint by image tiles: windowed marches of the
 //                rays that cross a tile, w_m * length summed in LDS in 64-bit
 //                fixed point, one float atomic per voxel at the end.
@@ -607,6 +611,442 @@ __global__ __launch_bounds__(256) void k_trace_fwd_rot(TraceArgs a)
     }
 }
 
+// ------------------------------------------------ tracer, segment by segment
+//
+// k_trace_seg: orbits of R rays as k_trace_fwd_rot, but each loop iteration is
+// one segment of the lane's ray instead of one major step with its two
+// candidate segments.  Along u = the major coordinate in the direction of
+// travel, the segments after plane 0 end at the major planes u_k = u_0 + k D
+// and at the minor grid lines, whose crossings x_n = c0 + c1 n are linear in
+// the line index too, so the next end is the smaller of two products; the
+// minor cell moves by one per crossing and the major index comes from the
+// segment's middle.  A step's crossing is then no masked half of the wave's
+// work, and per ray-segment about half the instructions remain.
+//
+// Decisions are those of march_loop: a plane and a line closer than the
+// margin, a middle within it of a major grid line or a set-up decision within
+// it leave the orbit to k_trace_redo, which marches its rays one by one; the
+// tests are kept
+// as running extremes and looked at once, after the loop.  The host rules out
+// grids whose plane-to-plane middles lie on grid lines (seg_grid).
+//
+// A workgroup holds 64 neighbouring orbits, 16 channels of 4 views; each of its
+// kSegWaves waves runs one window of the march, so all lanes of a wave are at
+// about the same place and its gathers fall into few cache lines: requests to
+// L2 bound the tracer before the instructions do (64 channels of one view per
+// wave drift apart by rows: 0.44 ms where 16 x 4 take 0.30; 8 x 8 and 32 x 2
+// 0.31 and 0.32; eight windows of eight orbits, the split before, 0.53).  The
+// windows' sums meet in LDS, one ray of the orbits after the other.
+// 800 x 609, against k_trace_fwd_rot: u16 M = 6 512^2 0.53 -> 0.29 ms, M = 8
+// 0.62 -> 0.33; float M = 6 512^2 1.08 -> 0.48, 768^2 2.53 -> 0.95; one ray
+// per march (401 views) against k_trace_fwd 0.60 -> 0.24.
+constexpr int kSegWaves = 8;
+
+// Bytes per voxel of the tracer's work copies: the materials in use.
+template <int M, int DT>
+constexpr int seg_voxel()
+{
+    return DT == VCT_DENS_U16 ? 4 * ((M + 1) / 2) : 8 * ((M + 1) / 2);
+}
+
+// A workgroup's 64 orbits: kSegCh neighbouring channels of 64 / kSegCh
+// neighbouring base views.
+constexpr int kSegCh = 16, kSegViews = 64 / kSegCh;
+__host__ __device__ __forceinline__ void seg_orbit(int block, int lane, int W, int& view, int& ch)
+{
+    const int ct = (W + kSegCh - 1) / kSegCh, vt = block / ct;
+    view = vt * kSegViews + lane / kSegCh;
+    ch = (block - vt * ct) * kSegCh + lane % kSegCh;
+}
+
+template <int M, int DT, int R>
+struct SegSums {
+    static constexpr int NW = (M + 1) / 2;
+    static constexpr int VB = seg_voxel<M, DT>(), ND = VB / 4;
+    // u16: sums of the 32-bit words and of their high halves (SinkU16)
+    double accw[R][NW], acch[R][NW];
+    struct Vox {
+        uint32_t w[ND];
+    };
+    __device__ __forceinline__ void init()
+    {
+#pragma unroll
+        for (int k = 0; k < R; k++)
+#pragma unroll
+            for (int j = 0; j < NW; j++) accw[k][j] = acch[k][j] = 0.0;
+    }
+    static __device__ __forceinline__ Vox load(const char* base, uint32_t o)
+    {
+        Vox q;
+        const char* p = base + o;
+        if constexpr (ND % 4 == 0) {
+#pragma unroll
+            for (int j = 0; j < ND / 4; j++) {
+                const uint4 t = reinterpret_cast<const uint4*>(p)[j];
+                q.w[4 * j] = t.x; q.w[4 * j + 1] = t.y; q.w[4 * j + 2] = t.z; q.w[4 * j + 3] = t.w;
+            }
+        } else if constexpr (ND == 6) {  // 8-byte aligned voxels
+            struct alignas(8) Six { uint32_t w[6]; };
+            const Six t = *reinterpret_cast<const Six*>(p);
+#pragma unroll
+            for (int j = 0; j < 6; j++) q.w[j] = t.w[j];
+        } else if constexpr (ND == 3) {
+            const uint3 t = *reinterpret_cast<const uint3*>(p);
+            q.w[0] = t.x; q.w[1] = t.y; q.w[2] = t.z;
+        } else if constexpr (ND == 2) {
+            const uint2 t = *reinterpret_cast<const uint2*>(p);
+            q.w[0] = t.x; q.w[1] = t.y;
+        } else {
+            q.w[0] = *reinterpret_cast<const uint32_t*>(p);
+        }
+        return q;
+    }
+    __device__ __forceinline__ void add(int k, const Vox& q, double rr)
+    {
+        if constexpr (DT == VCT_DENS_U16) {
+#pragma unroll
+            for (int j = 0; j < NW; j++) {
+                // odd M: the last word's high half is not a material of this call
+                const uint32_t w = 2 * j + 1 < M ? q.w[j] : q.w[j] & 0xffffu;
+                accw[k][j] = __builtin_fma((double)w, rr, accw[k][j]);
+                if (2 * j + 1 < M) acch[k][j] = __builtin_fma((double)(q.w[j] >> 16), rr, acch[k][j]);
+            }
+        } else {
+            // (the work copies hold max(rho, 0))
+#pragma unroll
+            for (int j = 0; j < NW; j++) {
+                accw[k][j] = __builtin_fma((double)__uint_as_float(q.w[2 * j]), rr, accw[k][j]);
+                if (2 * j + 1 < M)
+                    acch[k][j] = __builtin_fma((double)__uint_as_float(q.w[2 * j + 1]), rr, acch[k][j]);
+            }
+        }
+    }
+    __device__ __forceinline__ void scale(double f)
+    {
+#pragma unroll
+        for (int k = 0; k < R; k++)
+#pragma unroll
+            for (int j = 0; j < NW; j++) {
+                accw[k][j] *= f;
+                acch[k][j] *= f;
+            }
+    }
+    // material m of ray k
+    __device__ __forceinline__ double sum(int k, int m) const
+    {
+        const int j = m >> 1;
+        if (m & 1) return acch[k][j];
+        if (DT == VCT_DENS_U16 && m + 1 < M) return accw[k][j] - 65536.0 * acch[k][j];
+        return accw[k][j];
+    }
+};
+
+template <int M, int DT, int R>
+__global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
+{
+    using Sums = SegSums<M, DT, R>;
+    constexpr int VB = Sums::VB;
+    __shared__ double part[kSegWaves][M][64];
+    __shared__ int cnt[64], redo[64];
+    const int lane = threadIdx.x & 63, piece = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int Vq = (R == 1 ? a.VT : a.V / R);
+    int view, ch;
+    seg_orbit(blockIdx.x, lane, a.W, view, ch);
+    const bool valid = view < Vq && ch < a.W;
+    if (piece == 0) {
+        cnt[lane] = 0;
+        redo[lane] = 0;
+    }
+    __syncthreads();
+    Sums sums;
+    sums.init();
+    RayConst r;
+    bool safe = false;
+    const bool hit = valid && setup_ray(a, view, ch, r, &safe);
+    bool bad = valid && !safe;
+    if (hit && safe) {
+        const double ai = r.ai, af = r.af, Lb = r.Lb, D = a.D;
+        const double kAB = r.dB / r.dA, kBA = r.dA / r.dB;
+        const double sec = sqrt(1.0 + kAB * kAB);
+        const double pha = af > ai ? 1.0 : -1.0;
+        // integer-cm start plane, M/reprojection_TOMO.cpp:115-119
+        const int ain = ((ai < 0 && af < ai) || (ai > 0 && af > ai)) ? trunc_i32(trunc_i32(ai) + pha) : trunc_i32(ai);
+        const double uain = pha * (double)ain;
+        const double sA = r.xmajor ? 1.0 : -1.0, nxm = (double)a.nxm;
+        // set-up decisions that a turned ray might take otherwise, and slopes
+        // too small for the lines' crossings
+        bad = !((fabs(ai) == Lb || trunc_safe(ai)) && fabs(af - ai) >= kMarchMargin &&
+                fabs(r.bf - r.bi) >= kMarchMargin && fabs(kBA) <= 1.0e6);
+        // window of planes: this piece ends segments at planes k0 .. kstop
+        const int len = (march_step_estimate(a, r) + kSegWaves - 1) / kSegWaves;
+        const int k0 = max(piece * len, 1), k1 = piece == kSegWaves - 1 ? a.max_steps : (piece + 1) * len - 1;
+        // last plane inside the square (exactly u_0 + fl(k D) <= Lb)
+        int ka = (int)fmin(fmax((Lb - uain) / D, -1.0), 1.0e8);
+        if (uain + (double)(ka + 1) * D <= Lb) ka++;
+        if (ka >= 0 && uain + (double)ka * D > Lb) ka--;
+        const int kend = min(k1, ka + 1), kstop = min(kend, a.max_steps - 1);
+        // minor index value of plane k0 - 1: the cell and the first line ahead
+        const double u_start = uain + (double)(k0 - 1) * D;
+        const double b0 = __builtin_fma(pha * u_start - r.sa, kAB, r.sb);
+        const double hB = -sA * a.invD;
+        const double qb = __builtin_fma(b0, hB, nxm), fb = floor(qb);
+        // the general march's margins: 1e-9 voxel, and 1e-9 cm where it is the
+        // larger (a line is also where it compares signs and the square's edge)
+        const double margin = kMarchMargin * fmax(1.0, a.invD);
+        bad = bad || !(fabs(qb - fb - 0.5) < 0.5 - margin);
+        const bool up = (r.bf > r.bi) == (sA < 0.0);  // the minor index grows
+        const int dm = up ? 1 : -1;
+        int mi = (int)fmin(fmax(fb, -2.0), (double)a.N + 1.0);
+        double nd = (double)(up ? mi + 1 : mi) - nxm;  // next line, counted from the centre
+        const double c1 = pha * kBA * (-sA * D), c0 = pha * (r.sa - r.sb * kBA);
+        // each further line lies ahead, at least about a pitch on (|slope| <= 1),
+        // so the loop below ends
+        bad = bad || !(c1 * (double)dm > 0.5 * D);
+        const double hA = 0.5 * sA * pha * a.invD, q2 = nxm + 2.0;
+        // byte offsets in the two copies: row (major) and column (minor) parts
+        // of a voxel and of its turned images; slots 1 and 3 read the other copy
+        const int NP = a.N + 4, row = VB * NP;
+        const uint32_t size = (uint32_t)(NP * NP) * (uint32_t)VB;
+        const uint32_t baseE = r.xmajor ? size : 0u, dO = r.xmajor ? 0u - size : size;
+        const uint32_t rT = (uint32_t)((a.N + 3) * row) + 2u * baseE, cT = (uint32_t)((a.N + 3) * VB);
+        const char* copies = reinterpret_cast<const char*>(a.dens_t);
+        int n = 0;
+        const int inside = 2 * a.nxm;  // minor cells 0 .. inside - 1 lie in the square
+        bool ovf = false;
+        if (piece == 0 && !bad) {
+            // step 0: one segment from the entry to plane 0 (up to 1 cm, not cut
+            // at grid lines); its indices from the reference's exact expressions,
+            // whose ties on the major axis turn with the ray when the entry lies
+            // on a major side of the square (march_loop's a_sym)
+            const double be = ((double)ain - r.sa) / r.dA * r.dB + r.sb;
+            if (ka >= 0 && (unsigned)mi < (unsigned)inside) {
+                if (a.max_steps < 1) ovf = true;
+                else {
+                    n = 1;
+                    const double rr = fabs((double)ain - ai);
+                    const double ta = sA * ((ai + (double)ain) * 0.5) / D, tb = -sA * ((r.bi + be) * 0.5) / D;
+                    const double qa = ta + nxm, qm = tb + nxm;
+                    const bool sure_a = fabs(fabs(qa - trunc(qa)) - 0.5) < 0.5 - kMarchMargin;
+                    const bool sure_b = fabs(fabs(qm - trunc(qm)) - 0.5) < 0.5 - kMarchMargin;
+                    if (rr != 0.0) {
+                        if (!sure_b || !(sure_a || fabs(ai) == Lb)) bad = true;
+                        // each ray takes fl(+-t + N/2) of its own axis and its trunc:
+                        // index t + N/2 and N/2 - t, here as voxel numbers
+                        const int pa = trunc_i32(ta + nxm), na = trunc_i32(-ta + nxm);
+                        const int pb = trunc_i32(tb + nxm), nb = trunc_i32(-tb + nxm);
+                        auto in = [&](int v) { return v >= 0 && v <= a.N - 1; };
+                        auto one = [&](int k, uint32_t base, int ma, int mb) {
+                            if (!in(ma) || !in(mb)) return;
+                            sums.add(k, Sums::load(copies, base + (uint32_t)((ma + 2) * row) + (uint32_t)((mb + 2) * VB)),
+                                     rr);
+                        };
+                        one(0, baseE, pa, pb);
+                        if constexpr (R == 2) one(1, baseE, na, nb);
+                        if constexpr (R == 4) {
+                            one(2, baseE, na, nb);
+                            one(1, baseE + dO, pa, nb);
+                            one(3, baseE + dO, na, pb);
+                        }
+                    }
+                }
+            }
+        }
+        // the window's first plane k0 - 1 must be in the square, as march_loop
+        // tests before each step
+        if (!bad && k0 - 1 <= ka && (unsigned)mi < (unsigned)inside) {
+            if (k0 >= a.max_steps) ovf = k0 <= k1;
+            else if (k0 <= kend) {
+                // after i segments nc of them ended at a line and i - nc at a plane;
+                // i is the same on every lane
+                const int T = kstop - k0;
+                const double uk0 = uain + (double)k0 * D, ux0 = __builtin_fma(nd, c1, c0), dux = c1 * (double)dm;
+                const double near = margin * D * fabs(kBA);
+                const int dc = dm * VB;
+                const uint32_t cin = (uint32_t)(inside * VB);
+                uint32_t cu = (uint32_t)((mi + 2) * VB);
+                double uold = u_start;
+                int nc = 0;
+                int i = 0;
+                bool unsure = false;
+                struct Pending {
+                    typename Sums::Vox q[R];
+                    double rr;
+                };
+                // segment i: its gathers are issued into p; true if it is the last
+                auto step = [&](Pending& p) {
+                    const int t = i - nc;
+                    const double uk = __builtin_fma((double)t, D, uk0), ux = __builtin_fma((double)nc, dux, ux0);
+                    const double unew = fmin(ux, uk);
+                    p.rr = unew - uold;
+                    const bool cross = ux < uk;
+                    unsure |= fabs(uk - ux) < near;
+                    // the middle's major index (+ 2, so truncation is floor), and its
+                    // distance from the grid lines
+                    const double qa = __builtin_fma(uold + unew, hA, q2);
+                    unsure |= fabs(__builtin_amdgcn_fract(qa) - 0.5) > 0.5 - kMarchMargin;
+                    uold = unew;
+                    // (clamped: what lies outside reads the zero border)
+                    const uint32_t ia = min((uint32_t)(int)qa, (uint32_t)(a.N + 3)), c = min(cu, cT);
+                    const uint32_t ra = __umul24(ia, (uint32_t)row) + baseE;
+                    p.q[0] = Sums::load(copies, ra + c);
+                    if constexpr (R >= 2) {
+                        const uint32_t rt = rT - ra, ct = cT - c;
+                        p.q[R == 4 ? 2 : 1] = Sums::load(copies, rt + ct);
+                        if constexpr (R == 4) {
+                            p.q[1] = Sums::load(copies, ra + dO + ct);
+                            p.q[3] = Sums::load(copies, rt + dO + c);
+                        }
+                    }
+                    // after a plane the march goes on while it lies in the square
+                    const bool out = cu - 2u * VB >= cin;
+                    const bool end = !cross && (t >= T || out);
+                    if (end && !out && kstop < kend) ovf = true;
+                    nc += cross ? 1 : 0;
+                    cu += (uint32_t)(cross ? dc : 0);
+                    i++;
+                    return end;
+                };
+                auto add = [&](const Pending& p) {
+#pragma unroll
+                    for (int k = 0; k < R; k++) sums.add(k, p.q[k], p.rr);
+                };
+                // a segment's voxels are added while the next one's are fetched, in
+                // two register sets in turn; four rays of more than 6 materials add
+                // each at once (the second set would take the kernel past 128
+                // registers: 0.33 against 0.39 ms at 512^2, u16, M = 8)
+                Pending p0, p1;
+                if constexpr (R == 4 && M > 6) {
+                    bool end = false;
+                    while (!end) {
+                        end = step(p0);
+                        add(p0);
+                    }
+                } else if (step(p0)) {
+                    add(p0);
+                } else {
+                    for (;;) {
+                        bool end = step(p1);
+                        add(p0);
+                        if (end) {
+                            add(p1);
+                            break;
+                        }
+                        end = step(p0);
+                        add(p1);
+                        if (end) {
+                            add(p0);
+                            break;
+                        }
+                    }
+                }
+                n += i;
+                bad = unsure;
+            }
+        }
+        // (the lengths above lack the factor sec)
+        sums.scale(sec);
+        if (ovf) atomicOr(a.err, 1);
+        if (!bad && n) atomicAdd(&cnt[lane], n);
+    }
+    if (bad) redo[lane] = 1;
+    // the windows' sums, ray k of the 64 orbits at a time: wave w adds and
+    // writes slots w, w + kSegWaves, .. of every orbit
+    const bool xmaj = hit && r.xmajor;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < M; m++) part[piece][m][lane] = sums.sum(k, m);
+        __syncthreads();
+        // slots 1 and 3 hold rays 3 and 1 when y is the base ray's major axis
+        const int ray_k = (R == 4 && (k & 1) && !xmaj) ? 4 - k : k;
+        if (valid && !redo[lane]) {
+            const int ray = (view + ray_k * Vq) * a.W + ch;
+            float* dst = a.L + (size_t)ray * 8;
+            for (int m = piece; m < 8; m += kSegWaves) {
+                double t = 0.0;
+                if (m < M) {
+#pragma unroll
+                    for (int w = 0; w < kSegWaves; w++) t += part[w][m][lane];
+                }
+                dst[m] = (float)(t * a.out_scale);
+            }
+            if (piece == 0 && a.counts) a.counts[ray] = cnt[lane];
+        }
+    }
+    if (piece == 0) {
+        const unsigned long long m = __ballot(valid && redo[lane]);
+        if (lane == 0) a.redo[blockIdx.x] = m;
+    }
+}
+
+// The rays of the orbits that k_trace_seg left (bit l of redo[w]: lane l of
+// workgroup w), each by its own march in the 64 windows of a wave (a kernel of
+// its own, so that the general march's registers do not count against the
+// segment loop's).  One workgroup, a wave per ray of an orbit, per 64 words;
+// they are nearly always all zero.
+template <int M, int DT, int R>
+__global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words)
+{
+    constexpr int P = 64;
+    using Sink = std::conditional_t<DT == VCT_DENS_U16, SinkU16<M>, SinkF32<M>>;
+    const int w0 = blockIdx.x * 64, lane = threadIdx.x & 63, Vq = (R == 1 ? a.VT : a.V / R);
+    const unsigned long long mine = w0 + lane < words ? a.redo[w0 + lane] : 0ull;
+    unsigned long long any = __ballot(mine != 0ull);
+    while (any) {
+        const int w = __ffsll((long long)any) - 1;
+        any &= any - 1;
+        unsigned long long m = __shfl(mine, w);
+        while (m) {
+            int v0, ch;
+            seg_orbit(w0 + w, __ffsll((long long)m) - 1, a.W, v0, ch);
+            m &= m - 1;
+            const int view = v0 + (int)(threadIdx.x >> 6) * Vq, piece = lane;
+            RayConst r;
+            Sink sink;
+            sink.init(a.dens);
+            int iks = 0;
+            bool ovf = false;
+            if (setup_ray(a, view, ch, r)) {
+                const int len = (march_step_estimate(a, r) + P - 1) / P;
+                const int k0 = piece * len, k1 = piece == P - 1 ? INT_MAX : k0 + len - 1;
+                iks = r.dB != 0.0 ? march_loop<true>(a, r, sink, ovf, k0, k1) : march_loop<false>(a, r, sink, ovf, k0, k1);
+            }
+            if (ovf) atomicOr(a.err, 1);
+            if constexpr (DT == VCT_DENS_U16) sink.finish();
+            float out[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < M; q++) out[q] = (float)(group_sum<P>(sink.acc[q]) * a.out_scale);
+            iks = group_sum<P>(iks);
+            if (piece == 0) {
+                const int ray = view * a.W + ch;
+                float4* dst = reinterpret_cast<float4*>(a.L) + (size_t)ray * 2;
+                dst[0] = make_float4(out[0], out[1], out[2], out[3]);
+                dst[1] = make_float4(out[4], out[5], out[6], out[7]);
+                if (a.counts) a.counts[ray] = iks;
+            }
+        }
+    }
+}
+
+// Whether k_trace_seg serves this geometry: the guarded march without the
+// r >= rmax test, 32-bit offsets into the two copies, and no start plane whose
+// plane-to-plane middles fall on a major grid line (u_0 integer, middles at
+// u_0/D + k + 1/2: a grid of 128 voxels on 51.2 cm has such planes at every
+// odd centimetre, and each of their steps would be undecided).
+static bool seg_grid(const TraceArgs& a, int vb)
+{
+    if (a.exact || a.rcheck || !a.dens_t || !a.redo) return false;
+    const double np = a.N + 4.0;
+    if (2.0 * np * np * vb >= 4294967296.0 || (double)vb * np >= 8388608.0) return false;
+    const int last = (int)((double)a.nxm * a.D) + 2;
+    for (int c = 0; c <= last; c++) {
+        const double f = (double)c * a.invD + 0.5;
+        if (fabs(f - nearbyint(f)) < 1.0e-6) return false;
+    }
+    return true;
+}
+
 // Adjoint by image tiles.  Workgroup (chunk, tile) takes the views of one
 // chunk and one TS^2 tile of the image; for each view it finds the channels
 // whose rays can cross the tile (box_channels), and each such ray runs only
@@ -975,11 +1415,20 @@ __global__ __launch_bounds__(256) void k_pack_f32(const float* __restrict__ src,
     d[1] = make_float4(r[4], r[5], r[6], r[7]);
 }
 
+// Zero path integrals (and counts) of n rays.
+__global__ __launch_bounds__(256) void k_trace_zero(float* __restrict__ L, int32_t* __restrict__ counts, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float4* d = reinterpret_cast<float4*>(L) + (size_t)i * 2;
+    d[0] = d[1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (counts) counts[i] = 0;
+}
+
 // One voxel of the tracer's work copies: the first VB bytes of a packed
-// voxel (VB = 12: the three words of u16 materials 0-5; 16: all four; 32:
-// eight floats).
+// voxel (two bytes per u16 material, four per float one, in whole pairs).
 template <int VB>
-struct alignas(VB % 16 == 0 ? 16 : 4) WorkVox {
+struct alignas(VB % 16 == 0 ? 16 : VB % 8 == 0 ? 8 : 4) WorkVox {
     uint32_t w[VB / 4];
 };
 
@@ -987,8 +1436,10 @@ struct alignas(VB % 16 == 0 ? 16 : 4) WorkVox {
 // padded by two voxels on every side (NP = N + 4 per row): yx[y + 2][x + 2]
 // and xy[x + 2][y + 2] hold voxel (x, y) for x, y in [-1, N - 1], index -1
 // reading voxel 0 as the reference's truncation does, and zeros elsewhere;
-// by 32 x 32 tiles of the padded grid through LDS.
-template <int IB, int VB>
+// by 32 x 32 tiles of the padded grid through LDS.  CLAMP: float densities
+// below zero (and NaN) as 0, which is what they contribute
+// (M/reprojection_TOMO.cpp:155), so the sums need no test.
+template <int IB, int VB, bool CLAMP>
 __global__ __launch_bounds__(256) void k_pack_copies(const char* __restrict__ in, WorkVox<VB>* __restrict__ yx,
                                                      WorkVox<VB>* __restrict__ xy, int N)
 {
@@ -1005,6 +1456,10 @@ __global__ __launch_bounds__(256) void k_pack_copies(const char* __restrict__ in
         for (int q = 0; q < VB / 4; q++) t.w[q] = 0u;
         if (y >= -1 && y < N && x >= -1 && x < N)
             t = *reinterpret_cast<const WorkVox<VB>*>(in + ((size_t)max(y, 0) * N + max(x, 0)) * IB);
+        if constexpr (CLAMP) {
+#pragma unroll
+            for (int q = 0; q < VB / 4; q++) t.w[q] = __float_as_uint(fmaxf(__uint_as_float(t.w[q]), 0.f));
+        }
         tile[j][tx] = t;
         if (pr < NP && pc < NP) yx[(size_t)pr * NP + pc] = t;
     }
@@ -1015,13 +1470,13 @@ __global__ __launch_bounds__(256) void k_pack_copies(const char* __restrict__ in
     }
 }
 
-template <int IB, int VB>
+template <int IB, int VB, bool CLAMP = false>
 static void launch_pack_copies(const TraceArgs& a, hipStream_t s)
 {
     const int NP = a.N + 4;
     const dim3 grid((unsigned)((NP + 31) / 32), (unsigned)((NP + 31) / 32));
     WorkVox<VB>* yx = reinterpret_cast<WorkVox<VB>*>(a.dens_t);
-    hipLaunchKernelGGL((k_pack_copies<IB, VB>), grid, dim3(256), 0, s, reinterpret_cast<const char*>(a.dens), yx,
+    hipLaunchKernelGGL((k_pack_copies<IB, VB, CLAMP>), grid, dim3(256), 0, s, reinterpret_cast<const char*>(a.dens), yx,
                        yx + (size_t)NP * NP, a.N);
 }
 
@@ -1040,12 +1495,42 @@ static void launch_trace_rot(const TraceArgs& a, hipStream_t s)
                        dim3(a.block), 0, s, a);
 }
 
+template <int M, int DT>
+static vct_status launch_trace_seg(const TraceArgs& a, hipStream_t s)
+{
+    launch_pack_copies<DT == VCT_DENS_U16 ? 16 : 32, seg_voxel<M, DT>(), DT == VCT_DENS_F32>(a, s);
+    const int base_views = a.rot > 1 ? a.V / a.rot : a.VT;
+    const dim3 grid((unsigned)(((base_views + kSegViews - 1) / kSegViews) * ((a.W + kSegCh - 1) / kSegCh)));
+    const dim3 block(64 * kSegWaves);
+    if (a.VT < a.V) {
+        // an odd count's last view is not traced
+        const size_t done = (size_t)a.VT * a.W, rest = (size_t)(a.V - a.VT) * a.W;
+        hipLaunchKernelGGL(k_trace_zero, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0, s, a.L + done * 8,
+                           a.counts ? a.counts + done : nullptr, (int)rest);
+    }
+    if (base_views > 0) {
+        const int words = (int)grid.x;
+        const dim3 rgrid((unsigned)((words + 63) / 64));
+#define VCT_SEG(RR)                                                                  \
+    hipLaunchKernelGGL((k_trace_seg<M, DT, RR>), grid, block, 0, s, a);              \
+    hipLaunchKernelGGL((k_trace_redo<M, DT, RR>), rgrid, dim3(64 * RR), 0, s, a, words);
+        if (a.rot == 4) { VCT_SEG(4) }
+        else if (a.rot == 2) { VCT_SEG(2) }
+        else { VCT_SEG(1) }
+#undef VCT_SEG
+    }
+    VCT_HIP(hipGetLastError());
+    return VCT_OK;
+}
+
 template <int M>
 static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint, hipStream_t s)
 {
     const dim3 block(a.block);
     const dim3 grid((a.n_rays + a.block - 1) / a.block);
     const bool whole = a.ray_offset == 0 && a.n_rays == a.V * a.W;
+    if (!adjoint && whole && seg_grid(a, dens_type == VCT_DENS_U16 ? seg_voxel<M, VCT_DENS_U16>() : seg_voxel<M, VCT_DENS_F32>()))
+        return dens_type == VCT_DENS_U16 ? launch_trace_seg<M, VCT_DENS_U16>(a, s) : launch_trace_seg<M, VCT_DENS_F32>(a, s);
     if (!adjoint && whole && (a.rot == 4 || a.rot == 2)) {
         if (a.V % a.rot != 0 || a.N % 2 != 0 || a.VT != a.V || a.exact || a.rcheck || !a.dens_t)
             return set_error(VCT_ERR_INTERNAL, "orbit trace with V %d, N %d", a.V, a.N);
@@ -1083,6 +1568,11 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
     }
     VCT_HIP(hipGetLastError());
     return VCT_OK;
+}
+
+size_t trace_redo_words(int V, int W)
+{
+    return (size_t)((V + kSegViews - 1) / kSegViews) * (size_t)((W + kSegCh - 1) / kSegCh);
 }
 
 vct_status launch_trace(const TraceArgs& a, int dens_type, int M, bool adjoint, hipStream_t s)
