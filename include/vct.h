@@ -195,12 +195,11 @@ vct_status vct_pack_densities_f32(vct_plan* plan, const float* d_dens, int M,
  * ray's segments of rho_m * length, g/cm^2, divided by xfactor).  Each ray
  * is traced once, independent of the spectrum.  d_counts (optional, int32
  * [V][W]) receives the reference's per-ray segment counter
- * (reprojection_sum, :195/:280).  The call first writes d_packed and its
- * transpose, each padded by two voxels, into a work buffer that the plan
- * allocates with itself (64*(N+4)^2 bytes and a bit per ray), so that the
- * gathers of rays along x read rows too; calls on one plan must not overlap.
- * The exact option and geometries where the reference's r >= rmax test can
- * fire read d_packed itself. */
+ * (reprojection_sum, :195/:280).  With orbits (VCT_OPT_TRACE_ORBIT), the
+ * call first writes d_packed and its transpose, each padded by two voxels,
+ * into a work buffer that the plan allocates with itself (64*(N+4)^2 bytes
+ * when N and V are even), so that the gathers of rays along x read rows
+ * too; such calls on one plan must not overlap. */
 vct_status vct_trace_paths(vct_plan* plan, const void* d_packed, int dens_type, int M,
                            float* d_L, int32_t* d_counts, void* stream);
 

@@ -387,17 +387,18 @@ vct_status vct_plan_create(vct_ctx* ctx, const vct_geometry* g, vct_plan** out)
     if (st == VCT_OK) st = plan_upload(coeff.data(), W * sizeof(double), (void**)&p->d_coeff);
     // the orbit tracer's work copies (any dens type), allocated with the
     // plan so that no trace call allocates
-    if (st == VCT_OK) {
-        // two padded copies of (N + 4)^2 voxels of up to 32 bytes, the redo bits
-        const size_t np = (size_t)g->recon_size + 4, copies = 2 * np * np * 32;
-        const size_t bytes = copies + trace_redo_words(V, W) * 8;
-        if (hipMalloc(&p->d_dens_t, bytes) != hipSuccess) {
+    auto work = [&](size_t bytes, void** d) {
+        if (st == VCT_OK && hipMalloc(d, bytes) != hipSuccess) {
             (void)hipGetLastError();
             st = set_error(VCT_ERR_NOMEM, "plan work copy of %zu bytes", bytes);
-        } else {
-            p->d_redo = reinterpret_cast<unsigned long long*>(static_cast<char*>(p->d_dens_t) + copies);
         }
+    };
+    if (g->recon_size % 2 == 0 && V % 2 == 0) {
+        // two padded copies of (N + 4)^2 voxels of up to 32 bytes
+        const size_t np = (size_t)g->recon_size + 4;
+        work(2 * np * np * 32, &p->d_dens_t);
     }
+    work(trace_redo_words(V, W) * 8, (void**)&p->d_redo);
     if (st != VCT_OK) {
         vct_plan_destroy(p);
         return st;
@@ -452,6 +453,7 @@ vct_status vct_plan_destroy(vct_plan* p)
     for (float* b : p->d_toep)
         if (b) (void)hipFree(b);
     if (p->d_dens_t) (void)hipFree(p->d_dens_t);
+    if (p->d_redo) (void)hipFree(p->d_redo);
     delete p;
     return VCT_OK;
 }

@@ -178,8 +178,8 @@ struct vct_plan {
     double* d_coeff = nullptr;
     float* d_bpk[3] = {nullptr, nullptr, nullptr};   // packed filter matrix per type
     float* d_toep[3] = {nullptr, nullptr, nullptr};  // Toeplitz generator per type
-    void* d_dens_t = nullptr;  // the tracer's density work copies, then its redo bits
-    unsigned long long* d_redo = nullptr;  // inside d_dens_t
+    void* d_dens_t = nullptr;  // the orbit tracer's density work copies (N, V even)
+    unsigned long long* d_redo = nullptr;  // the tracer's redo bits
     int exact_trace = 0;  // VCT_OPT_EXACT_TRACE
     int max_steps = 0;    // VCT_OPT_MAX_STEPS (0: the automatic bound)
     int exact_bp = 0;     // VCT_OPT_EXACT_BACKPROJECT

@@ -639,7 +639,10 @@ __global__ __launch_bounds__(256) void k_trace_fwd_rot(TraceArgs a)
 // windows' sums meet in LDS, one ray of the orbits after the other.
 // 800 x 609, against k_trace_fwd_rot: u16 M = 6 512^2 0.53 -> 0.29 ms, M = 8
 // 0.62 -> 0.33; float M = 6 512^2 1.08 -> 0.48, 768^2 2.53 -> 0.95; one ray
-// per march (401 views) against k_trace_fwd 0.60 -> 0.24.
+// per march (401 views) against k_trace_fwd 0.60 -> 0.28.  Orbits read the
+// plan's work copies; one ray per march reads the packed densities, so that
+// calls of such a plan (odd views or grid) on several streams stay apart: the
+// redo bits, which all calls share, depend on the geometry alone.
 constexpr int kSegWaves = 8;
 
 // Bytes per voxel of the tracer's work copies: the materials in use.
@@ -662,7 +665,8 @@ __host__ __device__ __forceinline__ void seg_orbit(int block, int lane, int W, i
 template <int M, int DT, int R>
 struct SegSums {
     static constexpr int NW = (M + 1) / 2;
-    static constexpr int VB = seg_voxel<M, DT>(), ND = VB / 4;
+    // bytes of a voxel in the work copies (R == 1: a unit of the minor index)
+    static constexpr int ND = seg_voxel<M, DT>() / 4, VB = R == 1 ? 1 : 4 * ND;
     // u16: sums of the 32-bit words and of their high halves (SinkU16)
     double accw[R][NW], acch[R][NW];
     struct Vox {
@@ -712,12 +716,13 @@ struct SegSums {
                 if (2 * j + 1 < M) acch[k][j] = __builtin_fma((double)(q.w[j] >> 16), rr, acch[k][j]);
             }
         } else {
-            // (the work copies hold max(rho, 0))
+            // (a negative density contributes nothing, as SinkF32; the work
+            // copies hold max(rho, 0))
+            auto rho = [](uint32_t w) { return (double)(R == 1 ? fmaxf(__uint_as_float(w), 0.f) : __uint_as_float(w)); };
 #pragma unroll
             for (int j = 0; j < NW; j++) {
-                accw[k][j] = __builtin_fma((double)__uint_as_float(q.w[2 * j]), rr, accw[k][j]);
-                if (2 * j + 1 < M)
-                    acch[k][j] = __builtin_fma((double)__uint_as_float(q.w[2 * j + 1]), rr, acch[k][j]);
+                accw[k][j] = __builtin_fma(rho(q.w[2 * j]), rr, accw[k][j]);
+                if (2 * j + 1 < M) acch[k][j] = __builtin_fma(rho(q.w[2 * j + 1]), rr, acch[k][j]);
             }
         }
     }
@@ -809,7 +814,17 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
         const uint32_t size = (uint32_t)(NP * NP) * (uint32_t)VB;
         const uint32_t baseE = r.xmajor ? size : 0u, dO = r.xmajor ? 0u - size : size;
         const uint32_t rT = (uint32_t)((a.N + 3) * row) + 2u * baseE, cT = (uint32_t)((a.N + 3) * VB);
-        const char* copies = reinterpret_cast<const char*>(a.dens_t);
+        const char* copies = reinterpret_cast<const char*>(R == 1 ? a.dens : a.dens_t);
+        // R == 1: the packed densities themselves, by the ray's own axes
+        constexpr int IB = DT == VCT_DENS_U16 ? 16 : 32;
+        const int stA = (r.xmajor ? 1 : a.N) * IB, stB = (r.xmajor ? a.N : 1) * IB;
+        // voxel (ma, mb) of a lone ray, index -1 being 0 by truncation; outside
+        // the image the length is 0
+        auto lone = [&](int ma, int mb, double& rr) {
+            const bool in = (unsigned)(ma + 1) <= (unsigned)a.N && (unsigned)(mb + 1) <= (unsigned)a.N;
+            rr = in ? rr : 0.0;
+            return in ? (uint32_t)__umul24(max(ma, 0), stA) + (uint32_t)__umul24(max(mb, 0), stB) : 0u;
+        };
         int n = 0;
         const int inside = 2 * a.nxm;  // minor cells 0 .. inside - 1 lie in the square
         bool ovf = false;
@@ -840,7 +855,15 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
                             sums.add(k, Sums::load(copies, base + (uint32_t)((ma + 2) * row) + (uint32_t)((mb + 2) * VB)),
                                      rr);
                         };
-                        one(0, baseE, pa, pb);
+                        if constexpr (R == 1) {
+                            if (in(pa) && in(pb)) {
+                                double l = rr;
+                                const uint32_t o = lone(pa, pb, l);
+                                sums.add(0, Sums::load(copies, o), l);
+                            }
+                        } else {
+                            one(0, baseE, pa, pb);
+                        }
                         if constexpr (R == 2) one(1, baseE, na, nb);
                         if constexpr (R == 4) {
                             one(2, baseE, na, nb);
@@ -886,11 +909,13 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
                     unsure |= fabs(__builtin_amdgcn_fract(qa) - 0.5) > 0.5 - kMarchMargin;
                     uold = unew;
                     // (clamped: what lies outside reads the zero border)
-                    const uint32_t ia = min((uint32_t)(int)qa, (uint32_t)(a.N + 3)), c = min(cu, cT);
-                    const uint32_t ra = __umul24(ia, (uint32_t)row) + baseE;
-                    p.q[0] = Sums::load(copies, ra + c);
-                    if constexpr (R >= 2) {
+                    if constexpr (R == 1) {
+                        p.q[0] = Sums::load(copies, lone((int)qa - 2, (int)(cu / VB) - 2, p.rr));
+                    } else {
+                        const uint32_t ia = min((uint32_t)(int)qa, (uint32_t)(a.N + 3)), c = min(cu, cT);
+                        const uint32_t ra = __umul24(ia, (uint32_t)row) + baseE;
                         const uint32_t rt = rT - ra, ct = cT - c;
+                        p.q[0] = Sums::load(copies, ra + c);
                         p.q[R == 4 ? 2 : 1] = Sums::load(copies, rt + ct);
                         if constexpr (R == 4) {
                             p.q[1] = Sums::load(copies, ra + dO + ct);
@@ -1036,7 +1061,7 @@ __global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words)
 // odd centimetre, and each of their steps would be undecided).
 static bool seg_grid(const TraceArgs& a, int vb)
 {
-    if (a.exact || a.rcheck || !a.dens_t || !a.redo) return false;
+    if (a.exact || a.rcheck || !a.redo || (a.rot > 1 && !a.dens_t)) return false;
     const double np = a.N + 4.0;
     if (2.0 * np * np * vb >= 4294967296.0 || (double)vb * np >= 8388608.0) return false;
     const int last = (int)((double)a.nxm * a.D) + 2;
@@ -1498,7 +1523,7 @@ static void launch_trace_rot(const TraceArgs& a, hipStream_t s)
 template <int M, int DT>
 static vct_status launch_trace_seg(const TraceArgs& a, hipStream_t s)
 {
-    launch_pack_copies<DT == VCT_DENS_U16 ? 16 : 32, seg_voxel<M, DT>(), DT == VCT_DENS_F32>(a, s);
+    if (a.rot > 1) launch_pack_copies<DT == VCT_DENS_U16 ? 16 : 32, seg_voxel<M, DT>(), DT == VCT_DENS_F32>(a, s);
     const int base_views = a.rot > 1 ? a.V / a.rot : a.VT;
     const dim3 grid((unsigned)(((base_views + kSegViews - 1) / kSegViews) * ((a.W + kSegCh - 1) / kSegCh)));
     const dim3 block(64 * kSegWaves);
