@@ -923,18 +923,35 @@ __global__ __launch_bounds__(256) void k_bb_partial(BBArgs a)
     }
 }
 
-// alpha_b = clamp(sy > 0 ? ss / max(sy, 1e-30) : 2 alpha_b, 1e-8, 1e2)
-__global__ void k_bb_alpha(BBArgs a, int blocks)
+// alpha_b = clamp(sy > 0 ? ss / max(sy, 1e-30) : 2 alpha_b, 1e-8, 1e2), one
+// workgroup per phantom: lane t adds blocks t, t + 256, .. and the lanes meet
+// in a fixed tree (a serial loop over the blocks by one lane per phantom took
+// 0.24 ms of dependent loads for 16 phantoms, this 5 us).
+__global__ __launch_bounds__(256) void k_bb_alpha(BBArgs a, int blocks)
 {
-    const int b = threadIdx.x;
-    if (b >= a.B || a.first) return;
+    __shared__ double red[2][256];
+    const int b = blockIdx.x, t = threadIdx.x;
     double sy = 0.0, ss = 0.0;
-    for (int k = 0; k < blocks; k++) {
+    for (int k = t; k < blocks; k += 256) {
         sy += a.part[((size_t)k * a.B + b) * 2];
         ss += a.part[((size_t)k * a.B + b) * 2 + 1];
     }
-    const double bb = sy > 0.0 ? ss / fmax(sy, 1e-30) : 2.0 * (double)a.alpha[b];
-    a.alpha[b] = (float)fmin(fmax(bb, 1e-8), 1e2);
+    red[0][t] = sy;
+    red[1][t] = ss;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+        if (t < off) {
+            red[0][t] += red[0][t + off];
+            red[1][t] += red[1][t + off];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        sy = red[0][0];
+        ss = red[1][0];
+        const double bb = sy > 0.0 ? ss / fmax(sy, 1e-30) : 2.0 * (double)a.alpha[b];
+        a.alpha[b] = (float)fmin(fmax(bb, 1e-8), 1e2);
+    }
 }
 
 // x_prev = x, g_prev = g, x = max(x - alpha_b g, 0)
@@ -2324,7 +2341,7 @@ vct_status vct_batch_bb_step(float* d_x, float* d_x_prev, float* d_g_prev, const
     hipStream_t s = (hipStream_t)stream;
     if (!a.first) {
         hipLaunchKernelGGL(k_bb_partial, dim3(blocks), dim3(256), 0, s, a);
-        hipLaunchKernelGGL(k_bb_alpha, dim3(1), dim3(64), 0, s, a, blocks);
+        hipLaunchKernelGGL(k_bb_alpha, dim3(n_phantoms), dim3(256), 0, s, a, blocks);
     }
     hipLaunchKernelGGL(k_bb_apply, dim3(blocks), dim3(256), 0, s, a);
     VCT_HIP(hipGetLastError());
