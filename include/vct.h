@@ -130,7 +130,9 @@ vct_status vct_plan_destroy(vct_plan* plan);
  * sinogram is backprojected by orbits of the 90-degree rotation (pixel p
  * at view v + V/4 sees the geometry of pixel (y, N-1-x) at view v), which
  * computes each pixel-view geometry once for four pixels; its sums are in
- * another order (within 1e-5 relative of the reference's image).
+ * another order (within 1e-5 relative of the reference's image).  On other
+ * grids and view counts one sinogram's terms and sums are FP64, in orbits of
+ * the turns that the views allow, rounded to float once.
  * VCT_OPT_TRACE_ORBIT = 5: rays per march of vct_trace_paths: 4 (default)
  * marches the ray of view v once for the rays of views v + kV/4 (the same
  * segments turned by quarter turns, when V is a multiple of 4 and N even),

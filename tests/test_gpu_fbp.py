@@ -326,3 +326,25 @@ def test_multi_sinogram_float_weights_match_exact_terms(gpu, oracle, N, pix, V, 
         assert torch.equal(halves, fast)
     plan.close()
     exact_plan.close()
+
+
+@pytest.mark.parametrize("N,pix,V", [(65, 0.7, 84), (65, 0.7, 90), (64, 0.7, 90), (65, 0.7, 81), (64, 0.7, 83),
+                                      (127, 0.6, 90), (127, 0.6, 160), (8, 3.0, 6), (7, 3.0, 4), (9, 3.0, 2),
+                                      (17, 2.0, 3)])
+def test_single_sinogram_off_the_quarter_turn_grid(gpu, oracle, N, pix, V):
+    """One sinogram on odd grids and at view counts that are no multiple of
+    four (orbits of four, two or one pixels, the centre and the middle row of
+    odd grids, more waves than views): FP64 terms and sums, so the image is
+    the FP64 one rounded to float (half an ulp, 6e-8) but for the FP64
+    roundings of another operation order (below 1e-11 each); 0.6 cm pixels
+    take the library atan."""
+    ops = _ops()
+    g = Geom(N=N, pix=pix, V=V)
+    fl = np.random.default_rng(N * V).normal(size=(V, 609)).astype(np.float32) * 1e3
+    plan = ops.Plan(_geom(N, pix, V))
+    img = ops.backproject(plan, _t(fl, gpu))[0].cpu().numpy()
+    f64 = oracle.backproject_f64(g, fl.astype(np.float64))
+    scale = np.abs(f64).max()
+    assert np.all(np.abs(img - f64) <= 6.0e-8 * np.abs(f64) + 1.0e-9 * scale)
+    assert np.all(img[~oracle.mask(N).astype(bool)] == 0)
+    plan.close()
