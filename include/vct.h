@@ -311,6 +311,14 @@ vct_status vct_lengthproj_window(vct_plan* plan, const float* d_proj, int proj_w
  * single-sinogram call bit for bit. */
 vct_status vct_backproject(vct_plan* plan, const float* d_fltd, int n_sino, float* d_img,
                            void* stream);
+/* The same images bit for bit with a workspace of
+ * vct_backproject_workspace_bytes(plan, n_sino) bytes (0: none is used), in
+ * which several sinograms are interleaved in slices, at most 48 at a time, so
+ * that a lane reads its sinograms' taps in 16-byte loads.  d_work NULL:
+ * vct_backproject. */
+size_t vct_backproject_workspace_bytes(const vct_plan* plan, int n_sino);
+vct_status vct_backproject_ws(vct_plan* plan, const float* d_fltd, int n_sino, float* d_img, void* d_work,
+                              void* stream);
 /* The backprojections of n_groups (<= 16) geometries in one launch, as one
  * vct_backproject call per group (images bit-identical when the plans share
  * VCT_OPT_EXACT_BACKPROJECT; if any asks for it, all groups get exact

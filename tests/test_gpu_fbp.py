@@ -348,3 +348,25 @@ def test_single_sinogram_off_the_quarter_turn_grid(gpu, oracle, N, pix, V):
     assert np.all(np.abs(img - f64) <= 6.0e-8 * np.abs(f64) + 1.0e-9 * scale)
     assert np.all(img[~oracle.mask(N).astype(bool)] == 0)
     plan.close()
+
+
+@pytest.mark.parametrize("N,pix,V,S", [(512, 0.1, 90, 2), (512, 0.1, 90, 3), (300, 0.16, 91, 5), (200, 0.25, 90, 7),
+                                        (511, 0.1, 33, 9), (512, 0.1, 90, 12), (512, 0.1, 33, 13), (65, 0.7, 90, 23),
+                                        (300, 0.16, 33, 51), (128, 0.6, 160, 6), (16, 3.0, 2, 97), (16, 3.0, 1, 4)])
+def test_interleaved_slices_equal_plain_sinograms(gpu, N, pix, V, S):
+    """Several sinograms through interleaved slices (every width, padded last
+    slices, more than one pass of 48, the library atan) give the images of
+    the call without a workspace bit for bit."""
+    import torch
+    from virtualct_amd import _lib
+    ops = _ops()
+    plan = ops.Plan(_geom(N, pix, V))
+    fl = _t(np.random.default_rng(N + S).normal(size=(S, V, 609)).astype(np.float32) * 1e3, gpu)
+    for cap in (0, 2, 5, 16):
+        plan.set_option(_lib.OPT_BP_SINOS_PER_LANE, cap)
+        ref = torch.full((S, N, N), float("nan"), device=gpu)
+        torch.cuda.synchronize()
+        _lib.call("vct_backproject", plan.handle, fl.data_ptr(), S, ref.data_ptr(), None)
+        torch.cuda.synchronize()
+        assert torch.equal(ops.backproject(plan, fl), ref), cap
+    plan.close()

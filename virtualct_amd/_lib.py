@@ -90,6 +90,8 @@ _SIGS = {
     "vct_filter_workspace_bytes": (C.c_size_t, [_P, C.c_int]),
     "vct_filter_sinogram_ws": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, _P, _P, _P]),
     "vct_backproject": (C.c_int, [_P, _P, C.c_int, _P, _P]),
+    "vct_backproject_workspace_bytes": (C.c_size_t, [_P, C.c_int]),
+    "vct_backproject_ws": (C.c_int, [_P, _P, C.c_int, _P, _P, _P]),
     "vct_backproject_groups": (C.c_int, [_P, _P, _P, _P, C.c_int, C.c_int, _P]),
     "vct_interleaved_bytes": (C.c_size_t, [_P, C.c_int, C.c_int]),
     "vct_interleave_sinograms": (C.c_int, [_P, _P, C.c_int, C.c_int, _P, _P]),

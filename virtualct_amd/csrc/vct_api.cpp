@@ -795,6 +795,38 @@ vct_status vct_backproject(vct_plan* p, const float* d_fltd, int n_sino, float* 
     return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, pick_stream(p, stream));
 }
 
+// Sinograms that one pass of vct_backproject_ws interleaves (a bound on its
+// workspace).
+constexpr int kIlPass = 48;
+
+size_t vct_backproject_workspace_bytes(const vct_plan* p, int n_sino)
+{
+    if (!p || n_sino < 1) return 0;
+    const int K = bp_interleave_width(make_bp_args(p, nullptr, nullptr), n_sino);
+    if (K == 0) return 0;
+    const int n = std::min(n_sino, kIlPass / K * K);
+    return (size_t)((n + K - 1) / K) * K * p->g.n_views * p->g.n_channels * sizeof(float);
+}
+
+vct_status vct_backproject_ws(vct_plan* p, const float* d_fltd, int n_sino, float* d_img, void* d_work, void* stream)
+{
+    clear_error();
+    if (!p || !d_fltd || !d_img) return set_error(VCT_ERR_ARG, "NULL argument");
+    if (n_sino < 1 || n_sino > 65535) return set_error(VCT_ERR_ARG, "n_sino %d invalid", n_sino);
+    hipStream_t s = pick_stream(p, stream);
+    const int K = d_work ? bp_interleave_width(make_bp_args(p, nullptr, nullptr), n_sino) : 0;
+    if (K == 0) return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, s);
+    const int VW = p->g.n_views * p->g.n_channels;
+    const size_t NN = (size_t)p->g.recon_size * p->g.recon_size;
+    const int pass = kIlPass / K * K;
+    for (int i = 0; i < n_sino; i += pass) {
+        const int n = std::min(n_sino - i, pass);
+        VCT_CHECK(launch_interleave_sinos(d_fltd + (size_t)i * VW, n, VW, K, (float*)d_work, s));
+        VCT_CHECK(launch_backproject_il(make_bp_args(p, (const float*)d_work, d_img + i * NN), n, K, s));
+    }
+    return VCT_OK;
+}
+
 static vct_status backproject_groups(vct_plan* const* plans, const float* const* d_fltd, const int* n_sino,
                                      float* const* d_img, int n_groups, int sinos_per_lane, bool il, void* stream)
 {

@@ -235,6 +235,15 @@ __device__ __forceinline__ double rcp_f64(double x)
 static const double kAtanSym[kBpPoly] = {0.023298796324010433,  -0.05296597132474749, 0.07378028372611917,
                                          -0.09047114852983332,  0.1110744933786942,   -0.1428554012478447,
                                          0.19999995815529828,   -0.3333333329437766,  0.9999999999993997};
+// Largest |tan(gamma)| of a masked pixel, the tangent from the source to the
+// mask circle of radius r (pixel centres lie within mask_r pitches), beyond
+// the polynomials' range.
+static bool bp_wide(const BackprojArgs& a)
+{
+    const double r = a.mask_r * a.pix;
+    return !(r < a.sid) || r / std::sqrt(a.sid * a.sid - r * r) > 0.49;
+}
+
 static void set_poly(BackprojArgs& a)
 {
     for (int i = 0; i < kBpPoly; i++) a.poly[i] = kAtanSym[i] * a.inv_dbeta_ch;
@@ -367,14 +376,22 @@ __device__ __forceinline__ BpView bp_view(const BackprojArgs& a, double xx, doub
 // bp_view and applied in float, as in k_backproject_sym (within ~1e-6 of
 // the exact terms); otherwise every term is the single-sinogram FP64
 // expression and the images equal k_backproject's bit for bit.
-// IL (K a multiple of 4): a.fltd holds the sinograms interleaved in slices
-// of K, [S/K][V][W][K] (k_interleave_sinos), so the K tap pairs of a
-// pixel-view are 2K contiguous floats, read as K/2 16-byte loads instead of
-// 2K 4-byte ones; the same values, so the same images.
+// IL (K even): a.fltd holds the sinograms interleaved in slices of K,
+// [S/K][V][W][K] (k_interleave_sinos), so the K tap pairs of a pixel-view are
+// 2K contiguous floats, read as K/2 16-byte loads (8-byte aligned where K is
+// no multiple of 4) instead of 2K 4-byte ones; the same values, so the same
+// images.  Narrow slices leave registers for U views at once, whose geometry
+// chains and gathers overlap: each pixel adds its views one after the other,
+// so at 4 waves per SIMD and below the chain's latency bounds the kernel.  One
+// view per set -> U: K = 2 at 128^2 x 800 views 251 -> 143 us, K = 4 at 300^2
+// 215 -> 194, K = 12 at 768^2 1214 -> 1105; four per set lose what they gain
+// from K = 4 on (registers).  Wide slices are bound by the L1's 64 bytes per
+// clock: K = 12 at 512^2, 48 us per image.
 template <bool WIDE, int K, bool FW, bool IL = false>
 __device__ __forceinline__ void bp_multi_tile(const BackprojArgs& a, int S, int bx, int by, int bz)
 {
-    static_assert(!IL || K % 4 == 0, "interleaved slices hold a multiple of 4 sinograms");
+    constexpr int U = !IL || K > 12 ? 1 : K == 2 ? 4 : 2;
+    static_assert(!IL || K % 2 == 0, "interleaved slices hold an even number of sinograms");
     const double dbx = a.dbeta_view * a.xfactor;
     const int tx = threadIdx.x & (kBpTile - 1), ty = threadIdx.x / kBpTile;
     const int x = bx * kBpTile + tx;
@@ -391,12 +408,13 @@ __device__ __forceinline__ void bp_multi_tile(const BackprojArgs& a, int S, int 
         const uint32_t row = (uint32_t)(v * a.W);
         const uint32_t col = (uint32_t)g.col;
         if constexpr (IL) {
-            const float4* q = reinterpret_cast<const float4*>(slice + (size_t)row * K + col * (uint32_t)K);
+            struct alignas(K % 4 == 0 ? 16 : 8) Four { float v[4]; };
+            const Four* q = reinterpret_cast<const Four*>(slice + (size_t)row * K + col * (uint32_t)K);
 #pragma unroll
-            for (int h = 0; h < K / 4; h++) {
-                const float4 u = q[h], w = q[K / 4 + h];
-                t0[4 * h] = u.x; t0[4 * h + 1] = u.y; t0[4 * h + 2] = u.z; t0[4 * h + 3] = u.w;
-                t1[4 * h] = w.x; t1[4 * h + 1] = w.y; t1[4 * h + 2] = w.z; t1[4 * h + 3] = w.w;
+            for (int h = 0; h < K / 2; h++) {
+                const Four u = q[h];
+#pragma unroll
+                for (int j = 0; j < 4; j++) (4 * h + j < K ? t0[4 * h + j] : t1[4 * h + j - K]) = u.v[j];
             }
         } else {
 #pragma unroll
@@ -437,24 +455,36 @@ __device__ __forceinline__ void bp_multi_tile(const BackprojArgs& a, int S, int 
                 }
             }
         };
-        // two views per iteration in two register sets: view v + 1 is
-        // fetched while view v is summed, then view v + 2 while view v + 1
-        // is (no copies between the sets); an odd count's last fetch
-        // re-reads the last view and is not summed
+        // two sets of U views in registers: the next set is fetched while one
+        // is summed (no copies between them); what lies past the last view
+        // re-reads it and is not summed
+        struct Set {
+            BpView g[U];
+            float t0[U][K], t1[U][K];
+        };
         const int nv = a.use_views;
-        BpView g = bp_view<WIDE, FW>(a, xx, yy, 0), gn;
-        float r0[K], r1[K], n0[K], n1[K];
-        taps(0, g, r0, r1);
+        auto fetch = [&](Set& q, int v) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int w = min(v + u, nv - 1);
+                q.g[u] = bp_view<WIDE, FW>(a, xx, yy, w);
+                taps(w, q.g[u], q.t0[u], q.t1[u]);
+            }
+        };
+        auto sum = [&](const Set& q, int v) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (u == 0 || v + u < nv) add(q.g[u], q.t0[u], q.t1[u]);
+        };
+        Set p, q;
+        fetch(p, 0);
 #pragma unroll 1
-        for (int v = 0; v < nv; v += 2) {
-            const int v1 = min(v + 1, nv - 1), v2 = min(v + 2, nv - 1);
-            gn = bp_view<WIDE, FW>(a, xx, yy, v1);
-            taps(v1, gn, n0, n1);
-            add(g, r0, r1);
-            if (v + 1 == nv) break;
-            g = bp_view<WIDE, FW>(a, xx, yy, v2);
-            taps(v2, g, r0, r1);
-            add(gn, n0, n1);
+        for (int v = 0; v < nv; v += 2 * U) {
+            fetch(q, v + U);
+            sum(p, v);
+            if (v + U >= nv) break;
+            fetch(p, v + 2 * U);
+            sum(q, v + U);
         }
     }
     if (in_img) {
@@ -464,10 +494,10 @@ __device__ __forceinline__ void bp_multi_tile(const BackprojArgs& a, int S, int 
     }
 }
 
-template <bool WIDE, int K, bool FW>
+template <bool WIDE, int K, bool FW, bool IL = false>
 __global__ __launch_bounds__(kBpTile * kBpTile) void k_backproject_multi(BackprojArgs a, int S)
 {
-    bp_multi_tile<WIDE, K, FW>(a, S, blockIdx.x, blockIdx.y, blockIdx.z);
+    bp_multi_tile<WIDE, K, FW, IL>(a, S, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Several geometries in one launch: workgroup l belongs to the group g with
@@ -489,7 +519,8 @@ __global__ __launch_bounds__(kBpTile * kBpTile) void k_backproject_groups(BpGrou
 
 // Sinograms [S][VW] -> slices of K, dst[S/K][VW][K] (zeros past S): lane p
 // of slice sl gathers the K values of pixel-row entry p (each read coalesced
-// over the lanes) and stores them as K/4 16-byte stores.
+// over the lanes) and stores them as 16-byte (K a multiple of 4) or 8-byte
+// stores.
 template <int K>
 __global__ __launch_bounds__(256) void k_interleave_sinos(const float* __restrict__ src, int S, int VW,
                                                           float* __restrict__ dst)
@@ -502,9 +533,15 @@ __global__ __launch_bounds__(256) void k_interleave_sinos(const float* __restric
         const int s = sl * K + k;
         v[k] = s < S ? src[(size_t)s * VW + p] : 0.f;
     }
-    float4* d = reinterpret_cast<float4*>(dst + ((size_t)sl * VW + p) * K);
+    float* d = dst + ((size_t)sl * VW + p) * K;
+    if constexpr (K % 4 == 0) {
 #pragma unroll
-    for (int h = 0; h < K / 4; h++) d[h] = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+        for (int h = 0; h < K / 4; h++)
+            reinterpret_cast<float4*>(d)[h] = make_float4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
+    } else {
+#pragma unroll
+        for (int h = 0; h < K / 2; h++) reinterpret_cast<float2*>(d)[h] = make_float2(v[2 * h], v[2 * h + 1]);
+    }
 }
 
 // One sinogram by orbits of the quarter turn.  With V views over 360 degrees
@@ -808,8 +845,7 @@ vct_status launch_backproject_groups(BpGroups& ga, int K, hipStream_t s, bool il
         const BackprojArgs& a = ga.a[g];
         exact = exact || a.exact;
         if (ga.S[g] < 1) return set_error(VCT_ERR_ARG, "group %d has no sinograms", g);
-        const double r = a.mask_r * a.pix;
-        wide = wide || !(r < a.sid) || r / std::sqrt(a.sid * a.sid - r * r) > 0.49;
+        wide = wide || bp_wide(a);
         ga.tiles_x[g] = (a.N + kBpTile - 1) / kBpTile;
         total += (long long)ga.tiles_x[g] * ga.tiles_x[g] * ((ga.S[g] + K - 1) / K);
         if (total > INT_MAX) return set_error(VCT_ERR_ARG, "grouped backprojection too large");
@@ -842,12 +878,52 @@ vct_status launch_interleave_sinos(const float* src, int S, int VW, int K, float
     if (S < 1 || VW < 1) return set_error(VCT_ERR_ARG, "empty sinograms");
     const dim3 grid((VW + 255) / 256, (S + K - 1) / K), blk(256);
     switch (K) {
+    case 2: hipLaunchKernelGGL(k_interleave_sinos<2>, grid, blk, 0, s, src, S, VW, dst); break;
     case 4: hipLaunchKernelGGL(k_interleave_sinos<4>, grid, blk, 0, s, src, S, VW, dst); break;
+    case 6: hipLaunchKernelGGL(k_interleave_sinos<6>, grid, blk, 0, s, src, S, VW, dst); break;
     case 8: hipLaunchKernelGGL(k_interleave_sinos<8>, grid, blk, 0, s, src, S, VW, dst); break;
+    case 10: hipLaunchKernelGGL(k_interleave_sinos<10>, grid, blk, 0, s, src, S, VW, dst); break;
     case 12: hipLaunchKernelGGL(k_interleave_sinos<12>, grid, blk, 0, s, src, S, VW, dst); break;
     case 16: hipLaunchKernelGGL(k_interleave_sinos<16>, grid, blk, 0, s, src, S, VW, dst); break;
-    default: return set_error(VCT_ERR_ARG, "interleaved slices of %d sinograms (4, 8, 12 or 16)", K);
+    default: return set_error(VCT_ERR_ARG, "interleaved slices of %d sinograms (2, 4 .. 12 or 16)", K);
     }
+    VCT_HIP(hipGetLastError());
+    return VCT_OK;
+}
+
+// Width of the interleaved slices that S sinograms take, 0 for none (a single
+// sinogram, the exact option).  The fewest slices of at most 12, but enough
+// that the launch has kBpIlLanes lanes, and then the narrowest width that
+// holds an even share.  Measured (us, one launch, 800 views): 16 sinograms at
+// 512^2 as 3 x 6, 2 x 8, 12 + 4 and 1 x 16 867, 889, 1103 and 1235; 12 at
+// 300^2 as 2 x 6, 12 and 3 x 4 291, 319 and 363; 12 at 200^2 x 360 views as
+// 3 x 4, 2 x 6, 12 and 6 x 2 104, 114, 117 and 148.
+int bp_interleave_width(const BackprojArgs& a, int S)
+{
+    constexpr long long kBpIlLanes = 1 << 17;
+    if (S < 2 || a.exact) return 0;
+    const long long px = (long long)a.N * a.N;
+    const int cap = a.max_k >= 2 && a.max_k < 12 ? a.max_k / 2 * 2 : 12;
+    const int slices = std::max((S + cap - 1) / cap, (int)std::min<long long>((S + 1) / 2, (kBpIlLanes + px - 1) / px));
+    return ((S + slices - 1) / slices + 1) / 2 * 2;
+}
+
+vct_status launch_backproject_il(const BackprojArgs& args, int S, int K, hipStream_t s)
+{
+    BackprojArgs a = args;
+    set_poly(a);
+    const dim3 grid((a.N + kBpTile - 1) / kBpTile, (a.N + kBpTile - 1) / kBpTile, (S + K - 1) / K),
+        blk(kBpTile * kBpTile);
+#define VCT_BP_IL(KK)                                                                                      \
+    case KK:                                                                                               \
+        if (bp_wide(a)) hipLaunchKernelGGL((k_backproject_multi<true, KK, true, true>), grid, blk, 0, s, a, S); \
+        else hipLaunchKernelGGL((k_backproject_multi<false, KK, true, true>), grid, blk, 0, s, a, S);      \
+        break;
+    switch (K) {
+        VCT_BP_IL(2) VCT_BP_IL(4) VCT_BP_IL(6) VCT_BP_IL(8) VCT_BP_IL(10) VCT_BP_IL(12)
+    default: return set_error(VCT_ERR_INTERNAL, "interleaved slices of %d sinograms", K);
+    }
+#undef VCT_BP_IL
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }
@@ -903,11 +979,7 @@ vct_status launch_backproject(const BackprojArgs& args, int S, hipStream_t s)
     BackprojArgs a = args;
     set_poly(a);
     if (S <= 0) return set_error(VCT_ERR_ARG, "no sinograms to backproject");
-    // largest |tan(gamma)| of a masked pixel: the tangent from the source to
-    // the mask circle of radius r (pixel centres lie within mask_r pitches)
-    const double r = a.mask_r * a.pix;
-    const bool wide = !(r < a.sid) || r / std::sqrt(a.sid * a.sid - r * r) > 0.49;
-    if (wide)
+    if (bp_wide(a))
         launch_bp_w<true>(a, S, s);
     else
         launch_bp_w<false>(a, S, s);
