@@ -551,16 +551,18 @@ __global__ __launch_bounds__(256) void k_interleave_sinos(const float* __restric
 // T^-k(p), k = 0..3, at views v + kQ (mod V):
 //   T^0 = (x, y), T^-1 = (N-1-y, x), T^-2 = (N-1-x, N-1-y), T^-3 = (y, N-1-x).
 // A workgroup holds 64 base pixels (an 8 x 8 tile of the quadrant); wave w
-// runs views v in [wQ, (w+1)Q) with the software pipeline of
-// k_backproject_multi, so each pixel's 4 partial sums (wave 0 .. 3) are added
-// in that order through LDS.  The geometry follows the single-sinogram
+// runs the w-th eighth of the base views with the software pipeline of
+// k_backproject_multi, and each pixel's partial sums are added in the waves'
+// order through LDS.  (Eight waves because a small grid's are few: against
+// four 128^2 x 800 views 50 -> 31 us, 200^2 x 360 24 -> 16; 512^2 107 -> 105.)  The geometry follows the single-sinogram
 // expression in FP64; the interpolation and distance weights of a term are
 // applied in float, and the order of the float sum differs from the
 // reference's ascending views (images within 1e-5 of the reference's).
+constexpr int kBpSymWaves = 8;
 template <bool WIDE>
-__global__ __launch_bounds__(256) void k_backproject_sym(BackprojArgs a)
+__global__ __launch_bounds__(64 * kBpSymWaves) void k_backproject_sym(BackprojArgs a)
 {
-    __shared__ float part[3][4][64];
+    __shared__ float part[kBpSymWaves - 1][4][64];
     // the view range is per wave: made scalar, so the four rows of a view
     // are scalar bases and their wrap a scalar test
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -574,8 +576,9 @@ __global__ __launch_bounds__(256) void k_backproject_sym(BackprojArgs a)
     const double xx = -(x - a.center) * a.pix;  // :52-53
     const double yy = -(y - a.center) * a.pix;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    const int vb = wave * Q, ve = vb + Q;
-    if (masked && Q > 0) {
+    const int len = (a.V + kBpSymWaves - 1) / kBpSymWaves;
+    const int vb = wave * len, ve = min(vb + len, a.V);
+    if (masked && vb < ve) {
         // rows of view v + kQ (mod V); vb + kQ < V + 3Q, one wrap at most (a
         // scalar base; V * W <= 2^28)
         auto row_of = [&](int v, int k) {
@@ -627,7 +630,9 @@ __global__ __launch_bounds__(256) void k_backproject_sym(BackprojArgs a)
         const int py[4] = {y, x, n1 - y, n1 - x};
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const float v = ((acc[k] + part[0][k][lane]) + part[1][k][lane]) + part[2][k][lane];
+            float v = acc[k];
+#pragma unroll
+            for (int w = 0; w < kBpSymWaves - 1; w++) v += part[w][k][lane];
             a.img[(size_t)py[k] * a.N + px[k]] = v;
         }
     }
@@ -954,7 +959,7 @@ static void launch_bp_w(const BackprojArgs& a, int S, hipStream_t s)
     if (S == 1 && !a.exact && a.V % 4 == 0 && a.N % 2 == 0 && a.use_views == a.V && a.N >= 2) {
         const int h = a.N / 2;
         const dim3 grid((h + 7) / 8, (h + 7) / 8);
-        hipLaunchKernelGGL(k_backproject_sym<WIDE>, grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k_backproject_sym<WIDE>, grid, dim3(64 * kBpSymWaves), 0, s, a);
         return;
     }
     if (S == 1 && !a.exact) {
