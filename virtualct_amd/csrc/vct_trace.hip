@@ -415,28 +415,112 @@ struct SinkTile {
     unsigned long long* acc;  // [M][TS][PITCH], int64 or (FIXED false) float in the same memory
     int x0, y0;
     bool xmajor;
-    float scale;  // 2^S (FIXED)
-    float w[M];
+    float w[M];  // (FIXED: times 2^S)
+    __device__ __forceinline__ void add_at(int off, float r)
+    {
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const float c = w[m] * r;
+            if constexpr (FIXED) {
+                const long long q = (long long)__float2int_rn(c);
+                atomicAdd(acc + off + m * PLANE, (unsigned long long)q);
+            } else {
+                atomicAdd(reinterpret_cast<float*>(acc) + off + m * PLANE, c);
+            }
+        }
+    }
     __device__ __forceinline__ void add_ab(int ia, int ib, double rr)
     {
         const int x = xmajor ? ia : ib, y = xmajor ? ib : ia;
         const uint32_t lx = (uint32_t)(x - x0), ly = (uint32_t)(y - y0);
-        if (lx < (uint32_t)TS && ly < (uint32_t)TS) {
-            const float r = (float)rr;
-            const int off = (int)(ly * PITCH + lx);
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                const float c = w[m] * r;
-                if constexpr (FIXED) {
-                    const long long q = (long long)__float2int_rn(c * scale);
-                    atomicAdd(acc + off + m * PLANE, (unsigned long long)q);
-                } else {
-                    atomicAdd(reinterpret_cast<float*>(acc) + off + m * PLANE, c);
-                }
-            }
-        }
+        if (lx < (uint32_t)TS && ly < (uint32_t)TS) add_at((int)(ly * PITCH + lx), (float)rr);
     }
 };
+
+// Steps k0..k1 (k0 >= 1) of ray r into a tile, one segment per loop iteration
+// as k_trace_seg forms them, for grids that seg_planes accepts.  The margin
+// tests are looked at after the loop; false: one failed, and the window has
+// been taken out of the tile again by the same loop with the weights negated
+// (the fixed-point sums are exact, so nothing of it remains), for the caller to
+// march it step by step.  w is left as it was or negated.
+template <int M>
+__device__ __forceinline__ bool seg_window(const TraceArgs& a, const RayConst& r, SinkTile<M, true>& sink, bool& ovf,
+                                           int k0, int k1)
+{
+    using Sink = SinkTile<M, true>;
+    const double ai = r.ai, af = r.af, Lb = r.Lb, D = a.D;
+    const double kAB = r.dB / r.dA, kBA = r.dA / r.dB;
+    const double sA = r.xmajor ? 1.0 : -1.0, nxm = (double)a.nxm;
+    const double pha = af > ai ? 1.0 : -1.0;
+    // integer-cm start plane, M/reprojection_TOMO.cpp:115-119
+    const int ain = ((ai < 0 && af < ai) || (ai > 0 && af > ai)) ? trunc_i32(trunc_i32(ai) + pha) : trunc_i32(ai);
+    const double uain = pha * (double)ain;
+    // last plane inside the square (exactly u_0 + fl(k D) <= Lb)
+    int ka = (int)fmin(fmax((Lb - uain) / D, -1.0), 1.0e8);
+    if (uain + (double)(ka + 1) * D <= Lb) ka++;
+    if (ka >= 0 && uain + (double)ka * D > Lb) ka--;
+    const int kend = min(k1, ka + 1), kstop = min(kend, a.max_steps - 1);
+    // plane k0 - 1: the minor cell and the first line ahead
+    const double u_start = uain + (double)(k0 - 1) * D;
+    const double b0 = __builtin_fma(pha * u_start - r.sa, kAB, r.sb);
+    const double qb = __builtin_fma(b0, -sA * a.invD, nxm), fb = floor(qb);
+    const double margin = kMarchMargin * fmax(1.0, a.invD);
+    const bool up = (r.bf > r.bi) == (sA < 0.0);  // the minor index grows
+    const int dm = up ? 1 : -1;
+    const int mi0 = (int)fmin(fmax(fb, -2.0), (double)a.N + 1.0);
+    const double c1 = pha * kBA * (-sA * D), c0 = pha * (r.sa - r.sb * kBA);
+    // (the last test bounds the loop: each further line lies ahead)
+    if (!(fabs(qb - fb - 0.5) < 0.5 - margin && fabs(af - ai) >= kMarchMargin && fabs(r.bf - r.bi) >= kMarchMargin &&
+          fabs(kBA) <= 1.0e6 && c1 * (double)dm > 0.5 * D))
+        return false;
+    const int inside = 2 * a.nxm;
+    // the window's first plane must be in the square, as march_loop tests
+    if (k0 - 1 > ka || (unsigned)mi0 >= (unsigned)inside || k0 > kend) return true;
+    if (k0 >= a.max_steps) {
+        ovf = true;
+        return true;
+    }
+    const int T = kstop - k0;
+    const double uk0 = uain + (double)k0 * D, dux = c1 * (double)dm;
+    const double ux0 = __builtin_fma((double)(up ? mi0 + 1 : mi0) - nxm, c1, c0);
+    const double near = margin * D * fabs(kBA), sec = sqrt(1.0 + kAB * kAB);
+    const double hA = 0.5 * sA * pha * a.invD, q2 = nxm + 2.0;
+    const int oA = r.xmajor ? sink.x0 : sink.y0, oB = r.xmajor ? sink.y0 : sink.x0;
+    const int stA = r.xmajor ? 1 : Sink::PITCH, stB = r.xmajor ? Sink::PITCH : 1;
+    for (int pass = 0;; pass++) {
+        bool unsure = false;
+        double uold = u_start;
+        int t = 0, nc = 0, mi = mi0;
+        for (;;) {
+            const double uk = __builtin_fma((double)t, D, uk0), ux = __builtin_fma((double)nc, dux, ux0);
+            const double unew = fmin(ux, uk);
+            const bool cross = ux < uk;
+            unsure |= fabs(uk - ux) < near;
+            // the middle's major index (+ 2, so truncation is floor)
+            const double qa = __builtin_fma(uold + unew, hA, q2);
+            unsure |= fabs(__builtin_amdgcn_fract(qa) - 0.5) > 0.5 - kMarchMargin;
+            const int ia = (int)qa - 2;
+            // index -1 is 0 by truncation; what lies beyond N - 1 is not stored
+            const int la = max(ia, 0) - oA, lb = max(mi, 0) - oB;
+            if (ia >= -1 && mi >= -1 && (unsigned)la < (unsigned)Sink::TS && (unsigned)lb < (unsigned)Sink::TS)
+                sink.add_at(la * stA + lb * stB, (float)((unew - uold) * sec));
+            uold = unew;
+            // after a plane the march goes on while it lies in the square
+            const bool out = (unsigned)mi >= (unsigned)inside;
+            if (!cross && (t >= T || out)) {
+                if (!out && kstop < kend) ovf = true;
+                break;
+            }
+            t += cross ? 0 : 1;
+            nc += cross ? 1 : 0;
+            mi += cross ? dm : 0;
+        }
+        if (pass == 1) return false;
+        if (!unsure) return true;
+#pragma unroll
+        for (int m = 0; m < M; m++) sink.w[m] = -sink.w[m];
+    }
+}
 
 // ---------------------------------------------------------------- kernels
 
@@ -1059,11 +1143,17 @@ __global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words)
 // plane-to-plane middles fall on a major grid line (u_0 integer, middles at
 // u_0/D + k + 1/2: a grid of 128 voxels on 51.2 cm has such planes at every
 // odd centimetre, and each of their steps would be undecided).
+static bool seg_planes(const TraceArgs& a);
 static bool seg_grid(const TraceArgs& a, int vb)
 {
-    if (a.exact || a.rcheck || !a.redo || (a.rot > 1 && !a.dens_t)) return false;
+    if (!a.redo || (a.rot > 1 && !a.dens_t)) return false;
     const double np = a.N + 4.0;
     if (2.0 * np * np * vb >= 4294967296.0 || (double)vb * np >= 8388608.0) return false;
+    return seg_planes(a);
+}
+static bool seg_planes(const TraceArgs& a)
+{
+    if (a.exact || a.rcheck) return false;
     const int last = (int)((double)a.nxm * a.D) + 2;
     for (int c = 0; c <= last; c++) {
         const double f = (double)c * a.invD + 0.5;
@@ -1098,7 +1188,7 @@ __device__ __forceinline__ void adj_weights(const TraceArgs& a, int ray, float (
 }
 
 template <int M>
-__global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, int ntiles, int cv, int per_xcd)
+__global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, int ntiles, int cv, int per_xcd, int seg)
 {
     using Fixed = SinkTile<M, true>;
     using Float = SinkTile<M, false>;
@@ -1200,13 +1290,24 @@ __global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, in
         if (!box_steps(a, r, x_lo, x_hi, y_lo, y_hi, k0, k1)) continue;
         const bool fast = r.dB != 0.0 && !a.rcheck && !a.exact;
         if (fixed) {
-            Fixed sink{acc, x0, y0, r.xmajor, scale, {}};
+            Fixed sink{acc, x0, y0, r.xmajor, {}};
 #pragma unroll
-            for (int m = 0; m < M; m++) sink.w[m] = w[m];
-            if (fast) march_loop<true>(a, r, sink, ovf, k0, k1);
+            for (int m = 0; m < M; m++) sink.w[m] = w[m] * scale;
+            // (the segment loop starts after the entry's step 0)
+            if (fast && seg) {
+                if (k0 == 0) {
+                    march_loop<true>(a, r, sink, ovf, 0, 0);
+                    k0 = 1;
+                }
+                if (k0 <= k1 && !seg_window<M>(a, r, sink, ovf, k0, k1)) {
+#pragma unroll
+                    for (int m = 0; m < M; m++) sink.w[m] = w[m] * scale;
+                    march_loop<true>(a, r, sink, ovf, k0, k1);
+                }
+            } else if (fast) march_loop<true>(a, r, sink, ovf, k0, k1);
             else march_loop<false>(a, r, sink, ovf, k0, k1);
         } else {
-            Float sink{acc, x0, y0, r.xmajor, 1.f, {}};
+            Float sink{acc, x0, y0, r.xmajor, {}};
 #pragma unroll
             for (int m = 0; m < M; m++) sink.w[m] = w[m];
             if (fast) march_loop<true>(a, r, sink, ovf, k0, k1);
@@ -1584,7 +1685,7 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
             nchunk = (a.VT + cv - 1) / cv;
             const int per_xcd = (ntiles * nchunk + 7) / 8;
             hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(256), 0, s, a, ntx, ntiles, cv,
-                               per_xcd);
+                               per_xcd, seg_planes(a) ? 1 : 0);
         }
     } else if (dens_type == VCT_DENS_U16) {
         hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_U16, true>), grid, block, 0, s, a);
