@@ -300,3 +300,30 @@ def test_tile_adjoint_scales_with_tiny_and_huge_weights(gpu):
     for f in (1e-30, 1e-20, 1e20, 1e30):
         got = ops.trace_adjoint(plan, w * f, 4).cpu().numpy().astype(np.float64) / f
         assert rel_max(got, base) < 1e-6, f
+
+
+@pytest.mark.parametrize("N,pix,V,M,views", [(96, 0.52, 90, 1, 0), (101, 0.49, 91, 2, 0), (380, 50.0 / 380, 50, 6, 0),
+                                              (33, 1.7, 24, 3, 0), (200, 0.25, 300, 8, 256), (129, 0.39, 60, 7, 5),
+                                              (128, 0.4, 33, 5, 0), (31, 0.4, 12, 4, 0)])
+def test_tile_adjoint_segments_equal_the_exact_march(gpu, N, pix, V, M, views):
+    """The segment loop of the tile adjoint (odd and even grids, odd view
+    counts, images smaller than a tile and larger than the field, 128 x 0.4 cm
+    whose plane middles meet grid lines at odd centimetres and which marches
+    step by step, the largest view chunk) against the exact-division march:
+    the same segments, whose lengths differ by FP64 roundings, rounded to 2^-30
+    of the largest contribution and added in another order of floats."""
+    import torch
+    from virtualct_amd import _lib
+    ops = _ops()
+    g = torch.Generator(device=gpu).manual_seed(N + V)
+    w = torch.zeros((V, 609, 8), device=gpu)
+    w[..., :M] = torch.rand((V, 609, M), generator=g, device=gpu) - 0.25
+    out = []
+    for exact in (0, 1):
+        plan = ops.Plan(_geom(N, pix, V))
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        plan.set_option(_lib.OPT_ADJOINT_VIEWS, views)
+        out.append(ops.trace_adjoint(plan, w, M).cpu().numpy().astype(np.float64))
+        plan.close()
+    assert rel_max(out[0], out[1]) < 1e-6
+    assert np.count_nonzero(out[1][..., :M]) > 0 and np.all(out[0][..., M:] == 0)

@@ -393,47 +393,48 @@ struct SinkRot {
 // w[m] * length to the tile's accumulator in LDS, [m][row][col] with a row
 // pitch of TS + 1 (a wave's lanes are adjacent channels of one view, which
 // meet a column of the tile at one step when x is the major axis).  FIXED:
-// the accumulator is 64-bit fixed point, each contribution rounded to an
+// the accumulator is 51-bit fixed point, each contribution rounded to an
 // integer after scaling by a power of two that keeps it below 2^30 in
-// magnitude; the sums are then exact (and independent of the order of the
-// adds), and ds_add_u64 runs about ten times faster than ds_add_f32 on
+// magnitude (and 2^19 of them in range); the sums are then exact (and
+// independent of the order of the adds), and ds_add_u64 runs about ten times faster than ds_add_f32 on
 // gfx950 (0.3 vs 3.4 lane-operations per clock per CU, measured).  The float
 // form serves workgroups whose weights are not all finite, so NaN and
 // infinity reach the gradient as with float sums.
-template <int M>
-constexpr int adj_tile()
-{
-    return M <= 6 ? 32 : 28;  // M x TS x (TS + 1) x 8 B of LDS stays near 50 KB
-}
+constexpr int kAdjTile = 32;
 constexpr int kAdjMaxViews = 256;  // views per workgroup
+constexpr int kAdjBlock = 512;
 
 template <int M, bool FIXED>
 struct SinkTile {
     static constexpr bool kAdd2 = false;
     static constexpr bool kAB = true;
-    static constexpr int TS = adj_tile<M>(), PITCH = TS + 1, PLANE = TS * PITCH;
+    // (a plane's padding moves the next one by eight banks)
+    static constexpr int TS = kAdjTile, PITCH = TS + 1, PLANE = (TS * PITCH + 31) / 32 * 32 + 4;
     unsigned long long* acc;  // [M][TS][PITCH], int64 or (FIXED false) float in the same memory
     int x0, y0;
     bool xmajor;
-    float w[M];  // (FIXED: times 2^S)
-    __device__ __forceinline__ void add_at(int off, float r)
+    double w[M];  // (FIXED: times 2^S)
+    // FIXED: w r + 1.5 2^52 holds the product rounded to an integer in its low
+    // bits, so one fused multiply-add makes the addend; the magic's own bits
+    // are multiples of 2^51 and leave the sum's low 51 bits (fixed_sum) alone.
+    static constexpr double kMagic = 6755399441055744.0;
+    static __device__ __forceinline__ long long fixed_sum(unsigned long long acc) { return (long long)(acc << 13) >> 13; }
+    __device__ __forceinline__ void add_at(int off, double r)
     {
 #pragma unroll
         for (int m = 0; m < M; m++) {
-            const float c = w[m] * r;
-            if constexpr (FIXED) {
-                const long long q = (long long)__float2int_rn(c);
-                atomicAdd(acc + off + m * PLANE, (unsigned long long)q);
-            } else {
-                atomicAdd(reinterpret_cast<float*>(acc) + off + m * PLANE, c);
-            }
+            if constexpr (FIXED)
+                atomicAdd(acc + off + m * PLANE,
+                          (unsigned long long)__double_as_longlong(__builtin_fma(w[m], r, kMagic)));
+            else
+                atomicAdd(reinterpret_cast<float*>(acc) + off + m * PLANE, (float)w[m] * (float)r);
         }
     }
     __device__ __forceinline__ void add_ab(int ia, int ib, double rr)
     {
         const int x = xmajor ? ia : ib, y = xmajor ? ib : ia;
         const uint32_t lx = (uint32_t)(x - x0), ly = (uint32_t)(y - y0);
-        if (lx < (uint32_t)TS && ly < (uint32_t)TS) add_at((int)(ly * PITCH + lx), (float)rr);
+        if (lx < (uint32_t)TS && ly < (uint32_t)TS) add_at((int)(ly * PITCH + lx), rr);
     }
 };
 
@@ -485,7 +486,9 @@ __device__ __forceinline__ bool seg_window(const TraceArgs& a, const RayConst& r
     const double ux0 = __builtin_fma((double)(up ? mi0 + 1 : mi0) - nxm, c1, c0);
     const double near = margin * D * fabs(kBA), sec = sqrt(1.0 + kAB * kAB);
     const double hA = 0.5 * sA * pha * a.invD, q2 = nxm + 2.0;
+    // tile coordinates; index -1 is 0 by truncation, so the tiles at 0 take it
     const int oA = r.xmajor ? sink.x0 : sink.y0, oB = r.xmajor ? sink.y0 : sink.x0;
+    const int loA = oA == 0 ? -1 : 0, loB = oB == 0 ? -1 : 0;
     const int stA = r.xmajor ? 1 : Sink::PITCH, stB = r.xmajor ? Sink::PITCH : 1;
     for (int pass = 0;; pass++) {
         bool unsure = false;
@@ -499,11 +502,10 @@ __device__ __forceinline__ bool seg_window(const TraceArgs& a, const RayConst& r
             // the middle's major index (+ 2, so truncation is floor)
             const double qa = __builtin_fma(uold + unew, hA, q2);
             unsure |= fabs(__builtin_amdgcn_fract(qa) - 0.5) > 0.5 - kMarchMargin;
-            const int ia = (int)qa - 2;
-            // index -1 is 0 by truncation; what lies beyond N - 1 is not stored
-            const int la = max(ia, 0) - oA, lb = max(mi, 0) - oB;
-            if (ia >= -1 && mi >= -1 && (unsigned)la < (unsigned)Sink::TS && (unsigned)lb < (unsigned)Sink::TS)
-                sink.add_at(la * stA + lb * stB, (float)((unew - uold) * sec));
+            // (what lies beyond N - 1 is not stored)
+            const int la = (int)qa - (oA + 2), lb = mi - oB;
+            if ((unsigned)(la - loA) < (unsigned)(Sink::TS - loA) && (unsigned)(lb - loB) < (unsigned)(Sink::TS - loB))
+                sink.add_at((int)(__umul24(max(la, 0), stA) + __umul24(max(lb, 0), stB)), (unew - uold) * sec);
             uold = unew;
             // after a plane the march goes on while it lies in the square
             const bool out = (unsigned)mi >= (unsigned)inside;
@@ -1175,6 +1177,12 @@ static bool seg_planes(const TraceArgs& a)
 // test).  Work items are dealt to XCDs (workgroup g runs on XCD g % 8) in
 // contiguous runs, tile fastest, so the workgroups of one XCD share view
 // chunks and read their rays' weights through one L2.
+// Instruction issue and the LDS atomics (3.4 lane-operations per clock and CU)
+// bound it.  Two workgroups of 512 lanes per CU within 128 registers instead
+// of three of 256 lanes with 135: 380^2 x 722 views, M = 6, 1.38 -> 1.16 ms,
+// M = 8 1.87 -> 1.28; the addend by one fused multiply-add 1.53 -> 1.38; the
+// segment loop 1.91 -> 1.53; larger tiles (40) 1.11, but 0.14 instead of 0.12
+// at 64^2.
 template <int M>
 __device__ __forceinline__ void adj_weights(const TraceArgs& a, int ray, float (&w)[M])
 {
@@ -1188,7 +1196,7 @@ __device__ __forceinline__ void adj_weights(const TraceArgs& a, int ray, float (
 }
 
 template <int M>
-__global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, int ntiles, int cv, int per_xcd, int seg)
+__global__ __launch_bounds__(kAdjBlock, 4) void k_trace_adj_tile(TraceArgs a, int ntx, int ntiles, int cv, int per_xcd, int seg)
 {
     using Fixed = SinkTile<M, true>;
     using Float = SinkTile<M, false>;
@@ -1271,9 +1279,10 @@ __global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, in
     if (fixed) {
         int e;
         frexpf(wl, &e);  // wl < 2^e, e >= -79
-        S = 30 - e;      // <= 109
+        // (2^19 rays' contributions stay within the sums' 51 bits)
+        S = 30 - e - max(0, 32 - __clz(total) - 19);  // <= 109
     }
-    const float scale = ldexpf(1.f, S);
+    const double scale = ldexp(1.0, S);
     bool ovf = false;
     for (int i = threadIdx.x; i < total; i += blockDim.x) {
         int view, ch;
@@ -1318,19 +1327,16 @@ __global__ __launch_bounds__(256) void k_trace_adj_tile(TraceArgs a, int ntx, in
     __syncthreads();
     const float* dens = reinterpret_cast<const float*>(a.dens);
     const double unscale = ldexp(1.0, -S);
-    for (int i = threadIdx.x; i < TS * TS; i += blockDim.x) {
-        const int lx = i % TS, ly = i / TS;
+    // (eight lanes per voxel, so that a wave's adds cover whole lines of grad)
+    for (int i = threadIdx.x; i < TS * TS * 8; i += blockDim.x) {
+        const int m = i & 7, lx = (i >> 3) % TS, ly = (i >> 3) / TS;
         const int x = x0 + lx, y = y0 + ly;
-        if (x >= a.N || y >= a.N) continue;
+        if (m >= M || x >= a.N || y >= a.N) continue;
         const size_t v = (size_t)y * a.N + x;
-        const int off = ly * PITCH + lx;
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            float val = fixed ? (float)((double)(long long)acc[off + m * PLANE] * unscale)
-                              : reinterpret_cast<const float*>(acc)[off + m * PLANE];
-            if (dens && !(dens[v * 8 + m] >= 0.f)) val = 0.f;
-            if (val != 0.f) unsafeAtomicAdd(a.grad + v * 8 + m, val);
-        }
+        const int off = ly * PITCH + lx + m * PLANE;
+        float val = fixed ? (float)((double)Fixed::fixed_sum(acc[off]) * unscale) : reinterpret_cast<const float*>(acc)[off];
+        if (dens && !(dens[v * 8 + m] >= 0.f)) val = 0.f;
+        if (val != 0.f) unsafeAtomicAdd(a.grad + v * 8 + m, val);
     }
 }
 
@@ -1676,15 +1682,18 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
         }
     } else if (adjoint) {
         if (a.VT > 0) {
-            // about 2048 workgroups: enough view chunks to fill the chip twice over
-            const int ntx = (a.N + adj_tile<M>() - 1) / adj_tile<M>();
+            // 2048 workgroups, four rounds of two per CU, and 4096 where their
+            // chunks keep eight views (380^2 x 722 views 1.16 -> 1.07 ms; 200^2 x
+            // 360, with four views each, 0.37 -> 0.41)
+            const int ntx = (a.N + kAdjTile - 1) / kAdjTile;
             const int ntiles = ntx * ntx;
-            int nchunk = std::max(1, std::min(a.VT, (2048 + ntiles - 1) / ntiles));
+            const int target = (long long)ntiles * a.VT >= 8 * 4096 ? 4096 : 2048;
+            int nchunk = std::max(1, std::min(a.VT, (target + ntiles - 1) / ntiles));
             int cv = std::min((a.VT + nchunk - 1) / nchunk, kAdjMaxViews);
             if (a.adj_views > 0) cv = std::min(a.adj_views, kAdjMaxViews);
             nchunk = (a.VT + cv - 1) / cv;
             const int per_xcd = (ntiles * nchunk + 7) / 8;
-            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(256), 0, s, a, ntx, ntiles, cv,
+            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, cv,
                                per_xcd, seg_planes(a) ? 1 : 0);
         }
     } else if (dens_type == VCT_DENS_U16) {
