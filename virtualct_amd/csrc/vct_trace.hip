@@ -526,11 +526,35 @@ __device__ __forceinline__ bool seg_window(const TraceArgs& a, const RayConst& r
 
 // ---------------------------------------------------------------- kernels
 
-template <int M, int DT, bool FAST>
+// Sum over the P lanes of a group (P a power of two dividing 64, groups
+// aligned): every lane of the group gets the same sum.
+template <int P>
+__device__ __forceinline__ double group_sum(double x)
+{
+#pragma unroll
+    for (int d = 1; d < P; d <<= 1) x += __shfl_xor(x, d);
+    return x;
+}
+template <int P>
+__device__ __forceinline__ int group_sum(int x)
+{
+#pragma unroll
+    for (int d = 1; d < P; d <<= 1) x += __shfl_xor(x, d);
+    return x;
+}
+
+// One ray per P lanes, each marching one window of its steps (P = 1: the whole
+// march, in the reference's order).  Small calls have too few rays to hide a
+// march's latency, and the march of the r >= rmax test divides at every step:
+// 64^2 x 80 views 75 us with P = 1, 44, 46 and 48 with 4, 8 and 16; 64^2 x 800
+// 298, 270, 292 and 351; 128^2 (51.2 cm) x 81 153, 67, 64 and 59.
+template <int M, int DT, int P>
 __global__ __launch_bounds__(256) void k_trace_fwd(TraceArgs a)
 {
-    const int local = blockIdx.x * blockDim.x + threadIdx.x;
-    if (local >= a.n_rays) return;
+    using Sink = std::conditional_t<DT == VCT_DENS_U16, SinkU16<M>, SinkF32<M>>;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int local = t / P, piece = t % P;
+    if (local >= a.n_rays) return;  // (all lanes of a ray)
     const int ray = a.ray_offset + local;
     const int view = ray / a.W;
     const int ch = ray - view * a.W;
@@ -538,22 +562,26 @@ __global__ __launch_bounds__(256) void k_trace_fwd(TraceArgs a)
     int iks = 0;
     if (view < a.VT) {
         bool ovf = false;
-        if (DT == VCT_DENS_U16) {
-            SinkU16<M> sink;
-            sink.init(a.dens);
-            iks = march_ray<FAST>(a, view, ch, sink, ovf);
-            sink.finish();
-#pragma unroll
-            for (int m = 0; m < M; m++) out[m] = (float)(sink.acc[m] * a.out_scale);
+        Sink sink;
+        sink.init(a.dens);
+        if constexpr (P == 1) {
+            iks = march_ray<true>(a, view, ch, sink, ovf);
         } else {
-            SinkF32<M> sink;
-            sink.init(a.dens);
-            iks = march_ray<FAST>(a, view, ch, sink, ovf);
-#pragma unroll
-            for (int m = 0; m < M; m++) out[m] = (float)(sink.acc[m] * a.out_scale);
+            RayConst r;
+            if (setup_ray(a, view, ch, r)) {
+                const int len = (march_step_estimate(a, r) + P - 1) / P;
+                const int k0 = piece * len, k1 = piece == P - 1 ? INT_MAX : k0 + len - 1;
+                iks = r.dB != 0.0 && !a.rcheck && !a.exact ? march_loop<true>(a, r, sink, ovf, k0, k1)
+                                                           : march_loop<false>(a, r, sink, ovf, k0, k1);
+            }
         }
+        if constexpr (DT == VCT_DENS_U16) sink.finish();
+#pragma unroll
+        for (int m = 0; m < M; m++) out[m] = (float)(group_sum<P>(sink.acc[m]) * a.out_scale);
+        iks = group_sum<P>(iks);
         if (ovf) atomicOr(a.err, 1);
     }
+    if (piece != 0) return;
     float4* dst = reinterpret_cast<float4*>(a.L) + (size_t)ray * 2;
     dst[0] = make_float4(out[0], out[1], out[2], out[3]);
     dst[1] = make_float4(out[4], out[5], out[6], out[7]);
@@ -587,23 +615,6 @@ __device__ __forceinline__ void trace_one(const TraceArgs& a, int view, int ch)
     dst[0] = make_float4(out[0], out[1], out[2], out[3]);
     dst[1] = make_float4(out[4], out[5], out[6], out[7]);
     if (a.counts) a.counts[ray] = iks;
-}
-
-// Sum over the P lanes of a group (P a power of two dividing 64, groups
-// aligned): every lane of the group gets the same sum.
-template <int P>
-__device__ __forceinline__ double group_sum(double x)
-{
-#pragma unroll
-    for (int d = 1; d < P; d <<= 1) x += __shfl_xor(x, d);
-    return x;
-}
-template <int P>
-__device__ __forceinline__ int group_sum(int x)
-{
-#pragma unroll
-    for (int d = 1; d < P; d <<= 1) x += __shfl_xor(x, d);
-    return x;
 }
 
 // Orbits of R rays: the base ray (view v < V/R, channel) is marched once and
@@ -1696,10 +1707,15 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
             hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, cv,
                                per_xcd, seg_planes(a) ? 1 : 0);
         }
+    } else if (!a.exact && a.n_rays <= INT_MAX / 8) {
+        // (the exact option keeps the reference's order of the sums)
+        const dim3 split((4 * a.n_rays + a.block - 1) / a.block);
+        if (dens_type == VCT_DENS_U16) hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_U16, 4>), split, block, 0, s, a);
+        else hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_F32, 4>), split, block, 0, s, a);
     } else if (dens_type == VCT_DENS_U16) {
-        hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_U16, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_U16, 1>), grid, block, 0, s, a);
     } else {
-        hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_F32, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((k_trace_fwd<M, VCT_DENS_F32, 1>), grid, block, 0, s, a);
     }
     VCT_HIP(hipGetLastError());
     return VCT_OK;
