@@ -370,3 +370,17 @@ def test_interleaved_slices_equal_plain_sinograms(gpu, N, pix, V, S):
         torch.cuda.synchronize()
         assert torch.equal(ops.backproject(plan, fl), ref), cap
     plan.close()
+
+
+@pytest.mark.parametrize("W,V,S", [(609, 800, 5), (609, 400, 8), (100, 800, 21), (300, 801, 9), (33, 800, 45)])
+def test_tall_filter_products_equal_single_sinograms(gpu, W, V, S):
+    """Strips of column tiles (last strips of one to four tiles, edge tiles
+    within a strip, rows that are no multiple of 32) sum each output in the
+    order of a single sinogram's product: the same bits."""
+    from virtualct_amd import default_geometry
+    ops = _ops()
+    plan = ops.plan_for(default_geometry(recon_size=64, pixel_cm=0.7, n_views=V, n_channels=W, iso_channel=W / 2.0))
+    p = _t(np.random.default_rng(W + S).uniform(0.02, 1.0, (S, V, W)).astype(np.float32), gpu)
+    many = ops.filter_sinogram(plan, p, 2).cpu().numpy()
+    for i in (0, S // 2, S - 1):
+        assert np.array_equal(many[i], ops.filter_sinogram(plan, p[i], 2)[0].cpu().numpy()), i

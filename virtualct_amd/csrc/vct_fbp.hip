@@ -94,105 +94,132 @@ __global__ __launch_bounds__(256) void k_filter_prep(FilterPrepArgs a)
     *out = make_float4(row[0], row[2], row[4], row[6]);
 }
 
-constexpr int kFiltWaves = 4;  // K quarters of one 32x32 output tile, one wave each
-constexpr int kFiltU = 10;     // quads (4 MFMA steps each) a lane loads one chunk ahead
+constexpr int kFiltWaves = 4;  // K quarters of an output tile, one wave each
+constexpr int kFiltU = 10;     // quads (4 MFMA steps each) of A that a lane loads one chunk ahead
+constexpr int kFiltStrip = 4;  // column tiles per workgroup of a tall product
 
-// One 32x32 output tile per workgroup; wave w sums the w-th quarter of K, and
-// the quarters meet in LDS in a fixed order.  Operands are the pre-packed
-// register order: lane l = i + 32*h holds row/column i at k = 8q + 2j + h in
-// element j of float4 q.  Every lane loads a whole chunk of kFiltU float4 of A
-// and B before the chunk's MFMAs run, so 20-40 loads are in flight per lane.
+// NT 32x32 output tiles side by side per workgroup; wave w sums the w-th quarter
+// of K of each, and the quarters meet in LDS in a fixed order.  Operands are the
+// pre-packed register order: lane l = i + 32*h holds row/column i at
+// k = 8q + 2j + h in element j of float4 q.  Every lane loads a whole chunk of
+// A (and, NT = 1, of B) before the last chunk's MFMAs run, so that 10 loads or
+// more are in flight per lane.
 //
 // B is the filter matrix.  For a column tile whose rows are not renormalised
 // (edge_lo < m < edge_hi) it is Toeplitz, B[k][m] = toep[m - k + Kp - 1]: the
-// workgroup copies the tile's window of the generator (Kp + 31 floats) into
-// LDS and reads B from there, so only the few edge tiles read the packed
-// matrix from memory.
+// workgroup copies its tiles' window of the generator into LDS and reads B
+// from there, so only the few edge tiles read the packed matrix from memory.
 //
-// Tiles are dealt to XCDs in contiguous row-major ranges (workgroup g runs on
-// XCD g % 8), so an XCD reads about an eighth of A, once, into its L2.
-__global__ __launch_bounds__(256) void k_filter_gemm(FilterGemmArgs a, int ct, int ntiles, int per_xcd)
+// NT = 1 for a single sinogram, whose 500 tiles of 80 MFMAs a wave need every
+// wave they can get; a tall product (stacked sinograms) re-read A once per column tile and
+// was bound by that, so there an A quad serves NT tiles.  Every output is the
+// same sum in the same order for any NT.  Prep and product of 96 and 12
+// sinograms of 800 x 609: NT = 1 1160 and 155 us, 2 1050 and 137, 4 926 and 123,
+// 5 963 and 141 (the product then at 80 TFLOP/s); below 2000 tiles one per workgroup
+// is as fast or faster (2 sinograms 32 and 31 us, 4 of 300 channels 23 and 27).
+//
+// Workgroups are dealt to XCDs in contiguous row-major ranges (workgroup g runs
+// on XCD g % 8), so an XCD reads about an eighth of A, once, into its L2.
+template <int NT>
+__global__ __launch_bounds__(64 * kFiltWaves) void k_filter_gemm(FilterGemmArgs a, int ct, int cs, int nitems, int per_xcd)
 {
-    extern __shared__ float tw[];  // Toeplitz window, Kp + 31 floats
-    __shared__ float part[kFiltWaves - 1][16][64];
+    constexpr int U = NT == 1 ? kFiltU : kFiltU / 2;
+    extern __shared__ float tw[];  // Toeplitz window, Kp + 32 NT - 1 floats
+    __shared__ float part[kFiltWaves][16][64];
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int tile = xcd * per_xcd + slot;
-    if (slot >= per_xcd || tile >= ntiles) return;  // the whole workgroup
-    const int tr = tile / ct, tc = tile - tr * ct;
+    const int item = xcd * per_xcd + slot;
+    if (slot >= per_xcd || item >= nitems) return;  // the whole workgroup
+    const int tr = item / cs, tc0 = (item - tr * cs) * NT;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int Q = a.Kp / 8, Qw = Q / kFiltWaves;
     const int qb = wave * Qw, qe = qb + Qw;
-    const bool toep = tc * 32 > a.edge_lo && tc * 32 + 31 < a.edge_hi;  // uniform over the workgroup
-    if (toep) {
-        for (int j = threadIdx.x; j < a.Kp + 31; j += blockDim.x) tw[j] = a.toep[32 * tc + j];
+    const int nt = min(NT, ct - tc0);
+    bool toep[NT], any = false;  // uniform over the workgroup
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        const int m0 = (tc0 + n) * 32;
+        toep[n] = n < nt && m0 > a.edge_lo && m0 + 31 < a.edge_hi;
+        any = any || toep[n];
+    }
+    if (any) {
+        for (int j = threadIdx.x; j < a.Kp - 1 + 32 * nt; j += blockDim.x) tw[j] = a.toep[32 * tc0 + j];
         __syncthreads();
     }
     const float4* A = reinterpret_cast<const float4*>(a.apk) + ((size_t)tr * Q) * 64 + lane;
-    const float4* B = reinterpret_cast<const float4*>(a.bpk) + ((size_t)tc * Q) * 64 + lane;
+    const float4* B = reinterpret_cast<const float4*>(a.bpk) + ((size_t)tc0 * Q) * 64 + lane;
     // window index of B[k = 0] for this lane: column m = 32 tc + (lane & 31), k = lane >> 5
     const int t0 = (lane & 31) - (lane >> 5) + a.Kp - 1;
-    floatx16 acc;
+    auto b_quad = [&](int n, int q) {
+        if (toep[n]) {
+            const int t = t0 + 32 * n - 8 * q;
+            return make_float4(tw[t], tw[t - 2], tw[t - 4], tw[t - 6]);
+        }
+        return B[((size_t)n * Q + q) * 64];
+    };
+    floatx16 acc[NT];
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.f;
-    float4 ca[kFiltU], cb[kFiltU];
+    for (int n = 0; n < NT; n++)
 #pragma unroll
-    for (int u = 0; u < kFiltU; u++) {
-        const int q = qb + u;
-        if (q < qe) {
-            ca[u] = A[(size_t)q * 64];
-            if (toep) {
-                const int t = t0 - 8 * q;
-                cb[u] = make_float4(tw[t], tw[t - 2], tw[t - 4], tw[t - 6]);
-            } else {
-                cb[u] = B[(size_t)q * 64];
+        for (int i = 0; i < 16; i++) acc[n][i] = 0.f;
+    auto quad = [&](floatx16& c, const float4& x, const float4& y) {
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, c, 0, 0, 0);
+    };
+    float4 ca[U], cb[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (qb + u < qe) {
+            ca[u] = A[(size_t)(qb + u) * 64];
+            if (NT == 1) cb[u] = b_quad(0, qb + u);
+        }
+    for (int qs = qb; qs < qe; qs += U) {
+        float4 na[U], nb[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (qs + U + u < qe) {
+                na[u] = A[(size_t)(qs + U + u) * 64];
+                if (NT == 1) nb[u] = b_quad(0, qs + U + u);
+            }
+        if constexpr (NT == 1) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (qs + u < qe) quad(acc[0], ca[u], cb[u]);
+        } else {
+#pragma unroll
+            for (int n = 0; n < NT; n++) {
+                if (n >= nt) break;
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (qs + u < qe) cb[u] = b_quad(n, qs + u);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (qs + u < qe) quad(acc[n], ca[u], cb[u]);
             }
         }
-    }
-    for (int qs = qb; qs < qe; qs += kFiltU) {
-        float4 na[kFiltU], nb[kFiltU];
 #pragma unroll
-        for (int u = 0; u < kFiltU; u++) {
-            const int q = qs + kFiltU + u;
-            if (q < qe) {
-                na[u] = A[(size_t)q * 64];
-                if (toep) {
-                    const int t = t0 - 8 * q;
-                    nb[u] = make_float4(tw[t], tw[t - 2], tw[t - 4], tw[t - 6]);
-                } else {
-                    nb[u] = B[(size_t)q * 64];
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kFiltU; u++) {
-            if (qs + u < qe) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u].x, cb[u].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u].y, cb[u].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u].z, cb[u].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ca[u].w, cb[u].w, acc, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kFiltU; u++) {
+        for (int u = 0; u < U; u++) {
             ca[u] = na[u];
-            cb[u] = nb[u];
+            if (NT == 1) cb[u] = nb[u];
         }
     }
-    if (wave > 0) {
+    // each wave adds and writes a quarter of the rows of a tile
 #pragma unroll
-        for (int i = 0; i < 16; i++) part[wave - 1][i][lane] = acc[i];
-    }
-    __syncthreads();
-    if (wave == 0) {
-        const int j = lane & 31;
-        const int col = tc * 32 + j;
+    for (int n = 0; n < NT; n++) {
+        if (n >= nt) break;
+        if (n > 0) __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int row_in = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-            const int row = tr * 32 + row_in;
-            float v = acc[i] + part[0][i][lane];
+        for (int i = 0; i < 16; i++) part[wave][i][lane] = acc[n][i];
+        __syncthreads();
+        const int col = (tc0 + n) * 32 + (lane & 31);
 #pragma unroll
-            for (int w = 1; w < kFiltWaves - 1; w++) v += part[w][i][lane];
+        for (int ii = 0; ii < 16 / kFiltWaves; ii++) {
+            const int i = wave * (16 / kFiltWaves) + ii;
+            const int row = tr * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+            float v = part[0][i][lane];
+#pragma unroll
+            for (int w = 1; w < kFiltWaves; w++) v += part[w][i][lane];
             if (a.in_mode && (v < 1000.0f || v > 300000.0f)) v = 0.f;  // :250-255
             if (row < a.R && col < a.W) a.out[(size_t)row * a.W + col] = v;
         }
@@ -801,9 +828,12 @@ vct_status launch_filter(const FilterPrepArgs& p, const FilterGemmArgs& g, hipSt
     const int ct = Wp / 32;
     const long long ntiles = (long long)(Rp / 32) * ct;
     if (ntiles > INT_MAX / 2) return set_error(VCT_ERR_ARG, "filter GEMM too large");
-    const int per_xcd = (int)((ntiles + 7) / 8);
-    const size_t lds = (size_t)(g.Kp + 31) * sizeof(float);
-    hipLaunchKernelGGL(k_filter_gemm, dim3(8 * per_xcd), dim3(64 * kFiltWaves), lds, s, g, ct, (int)ntiles, per_xcd);
+    const int nt = ntiles >= 2000 ? kFiltStrip : 1;
+    const int cs = (ct + nt - 1) / nt, nitems = Rp / 32 * cs, per_xcd = (nitems + 7) / 8;
+    const size_t lds = (size_t)(g.Kp + 32 * nt - 1) * sizeof(float);
+    const dim3 grid(8 * per_xcd), blk(64 * kFiltWaves);
+    if (nt == 1) hipLaunchKernelGGL(k_filter_gemm<1>, grid, blk, lds, s, g, ct, cs, nitems, per_xcd);
+    else hipLaunchKernelGGL(k_filter_gemm<kFiltStrip>, grid, blk, lds, s, g, ct, cs, nitems, per_xcd);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }
