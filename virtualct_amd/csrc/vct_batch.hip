@@ -50,6 +50,7 @@
 
 #include "vct_internal.h"
 #include "vct_march.h"
+#include "vct_spectral.h"
 
 // Two-stage form of one direction (see above).
 struct vct_blocked {
@@ -617,139 +618,40 @@ __device__ __forceinline__ void spec_slot(const BatchSpecArgs& a, int z, const f
     b = z - a.pref[g];
 }
 
-// One past the highest bin with a nonzero probability among the bins this
-// wave's lanes hold (bin e on this lane, consecutive bins on consecutive
-// lanes), or 0; called by every active lane, it needs no atomics.
-__device__ __forceinline__ int last_nonzero_bin(int e, float p)
-{
-    const unsigned long long m = __ballot(p != 0.f);
-    const int base = e - (int)(threadIdx.x & 63);  // the bin of lane 0
-    return m ? base + 64 - __clzll((long long)m) : 0;
-}
-
-// Forward mode: raw and per-(b,s) max/min, one (b,s) per blockIdx.y/z.
-// Launched with 256 threads (four waves).
-template <int M>
-__global__ __launch_bounds__(256) void k_batch_spectral(BatchSpecArgs a)
-{
-    extern __shared__ float lds[];
-    float* mu2 = lds;
-    float* pdf = lds + a.NE * 8;
-    __shared__ uint32_t red[2][4];
-    __shared__ int ne_w[4];
-    const int s = blockIdx.y, z = blockIdx.z, NE = a.NE;
-    const float* Lrows;
-    int B, b;
-    spec_slot(a, z, Lrows, B, b);
-    const float kLog2e = 1.4426950408889634f;
-    for (int i = threadIdx.x; i < NE * 8; i += blockDim.x) {
-        const int e = i >> 3, m = i & 7;
-        mu2[i] = (m < M) ? -a.att[((size_t)s * M + m) * NE + e] * kLog2e : 0.f;
-    }
-    // bins past the spectrum's last nonzero probability (the zero padding of
-    // spectra of unequal length) add exactly +0 and are skipped
-    int last = 0;
-    for (int e = threadIdx.x; e < NE; e += blockDim.x) {
-        const float p = a.pdf[(size_t)s * NE + e];
-        pdf[e] = p;
-        last = max(last, last_nonzero_bin(e, p));
-    }
-    if ((threadIdx.x & 63) == 0) ne_w[threadIdx.x >> 6] = last;
-    __syncthreads();
-    const int ne = max(max(ne_w[0], ne_w[1]), max(ne_w[2], ne_w[3]));
-    const int ray = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = ray < a.rays;
-    float I = 0.f;
-    if (valid && ray / a.W < a.VT) {
-        float Lm[8];
-        load_slot<M>(Lrows, ray, B, b, Lm);
-        for (int e = 0; e < ne; e++) {
-            const float4 m0 = reinterpret_cast<const float4*>(mu2)[2 * e];
-            const float4 m1 = reinterpret_cast<const float4*>(mu2)[2 * e + 1];
-            const float mu[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-            float x = 0.f;
-#pragma unroll
-            for (int m = 0; m < M; m++) x = fmaf(mu[m], Lm[m], x);
-            I += pdf[e] * __builtin_amdgcn_exp2f(x);  // as k_spectral
-        }
-    }
-    const size_t bs = (size_t)z * a.S + s;
-    if (valid) a.raw[bs * a.rays + ray] = I;
-    uint32_t mx = valid ? __float_as_uint(I) : 0u;
-    uint32_t mn = valid ? __float_as_uint(I) : 0x7f800000u;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
-        mn = min(mn, (uint32_t)__shfl_xor((int)mn, off, 64));
-    }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { red[0][wave] = mx; red[1][wave] = mn; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) { mx = max(mx, red[0][w]); mn = min(mn, red[1][w]); }
-        atomicMax(a.stats + 2 * bs, mx);
-        atomicMin(a.stats + 2 * bs + 1, mn);
-    }
-}
-
-// Forward mode with every spectrum of phantom blockIdx.z in one block: the
-// tables and the ray's path integrals are loaded once for all S spectra.
-// Each (phantom, spectrum, ray) is summed exactly as in k_batch_spectral.
-// Rays per workgroup of k_batch_spectral_all: each workgroup adds its max and
-// min of each (phantom, spectrum) to that pair's statistics words with one
-// atomic each, which serialise per address, so workgroups are large.
+// Forward mode: raw and per-(phantom, spectrum) max/min, all spectra of phantom
+// blockIdx.z, one after the other, in one block: the ray's path integrals are
+// loaded once, and the table of one spectrum at a time is in LDS (spec_sum).
+// Rays per workgroup: each workgroup adds its max and min of each (phantom,
+// spectrum) to that pair's statistics words with one atomic each, which
+// serialise per address, so workgroups are large.
 constexpr int kSpecAllBlock = 1024, kSpecAllWaves = kSpecAllBlock / 64;
 
+// Material m of slot (row, b) (see load_slot).
+__device__ __forceinline__ size_t slot_index(size_t row, int B, int b, int m)
+{
+    return row * (size_t)(8 * B) + (m < 4 ? 4 * b + m : (m & ~1) * B + 2 * b + (m & 1));
+}
+
 template <int M>
-__global__ __launch_bounds__(kSpecAllBlock) void k_batch_spectral_all(BatchSpecArgs a)
+__global__ __launch_bounds__(kSpecAllBlock) void k_batch_spectral(BatchSpecArgs a)
 {
     extern __shared__ float lds[];
     const int S = a.S, NE = a.NE, z = blockIdx.z;
     const float* Lrows;
     int B, b;
     spec_slot(a, z, Lrows, B, b);
-    float* mu2 = lds;                                          // [S][NE][8]
-    float* pdf = lds + (size_t)S * NE * 8;                     // [S][NE]
-    int* ne_w = reinterpret_cast<int*>(pdf + (size_t)S * NE);  // [S][kSpecAllWaves]
     __shared__ uint32_t red[2][kSpecAllWaves];
-    const float kLog2e = 1.4426950408889634f;
-    for (int i = threadIdx.x; i < S * NE * 8; i += blockDim.x) {
-        const int s = i / (NE * 8), r = i - s * NE * 8, e = r >> 3, m = r & 7;
-        mu2[i] = (m < M) ? -a.att[((size_t)s * M + m) * NE + e] * kLog2e : 0.f;
-    }
-    for (int s = 0; s < S; s++) {
-        int last = 0;
-        for (int e = threadIdx.x; e < NE; e += blockDim.x) {
-            const float p = a.pdf[(size_t)s * NE + e];
-            pdf[s * NE + e] = p;
-            last = max(last, last_nonzero_bin(e, p));
-        }
-        if ((threadIdx.x & 63) == 0) ne_w[kSpecAllWaves * s + (threadIdx.x >> 6)] = last;
-    }
-    __syncthreads();
-    const int ray = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int last[kSpecAllWaves];
+    const int ray = blockIdx.x * blockDim.x + threadIdx.x, ray0 = ray & ~63, traced = a.VT * a.W;
     const bool valid = ray < a.rays;
-    const bool hit = valid && ray / a.W < a.VT;
-    float Lm[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (hit) load_slot<M>(Lrows, ray, B, b, Lm);
+    SpecRays<M> L;
+    L.load([&](int t, int m) { return ray0 + t < traced ? Lrows[slot_index(ray0 + t, B, b, m)] : 0.f; });
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int s = 0; s < S; s++) {
-        int ne = 0;
-        for (int w = 0; w < kSpecAllWaves; w++) ne = max(ne, ne_w[kSpecAllWaves * s + w]);
-        const float* mus = mu2 + (size_t)s * NE * 8;
-        const float* ps = pdf + (size_t)s * NE;
-        float I = 0.f;
-        if (hit) {
-            for (int e = 0; e < ne; e++) {
-                const float4 m0 = reinterpret_cast<const float4*>(mus)[2 * e];
-                const float4 m1 = reinterpret_cast<const float4*>(mus)[2 * e + 1];
-                const float mu[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-                float x = 0.f;
-#pragma unroll
-                for (int m = 0; m < M; m++) x = fmaf(mu[m], Lm[m], x);
-                I += ps[e] * __builtin_amdgcn_exp2f(x);  // as k_spectral
-            }
-        }
+        const SpecTable<M> tab =
+            SpecTable<M>::fill(lds, last, a.att + (size_t)s * M * NE, a.pdf + (size_t)s * NE, NE);
+        float I = spec_sum<M>(tab, L);
+        if (ray >= traced) I = 0.f;
         const size_t bs = (size_t)z * S + s;
         if (valid) a.raw[bs * a.rays + ray] = I;
         uint32_t mx = valid ? __float_as_uint(I) : 0u;
@@ -766,7 +668,7 @@ __global__ __launch_bounds__(kSpecAllBlock) void k_batch_spectral_all(BatchSpecA
             atomicMax(a.stats + 2 * bs, mx);
             atomicMin(a.stats + 2 * bs + 1, mn);
         }
-        __syncthreads();  // red is reused by the next spectrum
+        __syncthreads();  // the table and red are reused by the next spectrum
     }
 }
 
@@ -2358,6 +2260,20 @@ static vct_status check_spec(vct_plan* p, const float* L, int B, int M, const fl
     return VCT_OK;
 }
 
+static void launch_batch_spectral(const BatchSpecArgs& a, int M, int B, hipStream_t s)
+{
+    const dim3 grid((a.rays + kSpecAllBlock - 1) / kSpecAllBlock, 1, B), blk(kSpecAllBlock);
+    switch (M) {
+#define VCT_SPEC_CASE(MM)                                                                                            \
+    case MM:                                                                                                         \
+        hipLaunchKernelGGL((k_batch_spectral<MM>), grid, blk, sizeof(float) * SpecTable<MM>::floats(a.NE), s, a); \
+        break;
+        VCT_SPEC_CASE(1) VCT_SPEC_CASE(2) VCT_SPEC_CASE(3) VCT_SPEC_CASE(4)
+        VCT_SPEC_CASE(5) VCT_SPEC_CASE(6) VCT_SPEC_CASE(7) VCT_SPEC_CASE(8)
+#undef VCT_SPEC_CASE
+    }
+}
+
 vct_status vct_batch_spectral(vct_plan* p, const float* d_L, int B, int M, const float* d_att, const float* d_pdf,
                               int NE, int S, float* d_raw, uint32_t* d_stats, void* stream)
 {
@@ -2370,29 +2286,7 @@ vct_status vct_batch_spectral(vct_plan* p, const float* d_L, int B, int M, const
     a.rays = p->g.n_views * p->g.n_channels; a.W = p->g.n_channels; a.VT = p->VT;
     a.B = B; a.S = S; a.M = M; a.NE = NE;
     hipLaunchKernelGGL(k_batch_stats_init, dim3((B * S + 63) / 64), dim3(64), 0, s, d_stats, B * S);
-    // all spectra of a phantom per block while their tables fit in 64 KB of
-    // LDS (two blocks per CU); else one (phantom, spectrum) per block
-    const size_t lds_all = sizeof(float) * (size_t)S * NE * 9 + sizeof(int) * kSpecAllWaves * S;
-    if (lds_all <= 64 * 1024) {
-        const dim3 grid((a.rays + kSpecAllBlock - 1) / kSpecAllBlock, 1, B);
-        switch (M) {
-#define VCT_SPEC_CASE(MM) \
-    case MM: hipLaunchKernelGGL((k_batch_spectral_all<MM>), grid, dim3(kSpecAllBlock), lds_all, s, a); break;
-            VCT_SPEC_CASE(1) VCT_SPEC_CASE(2) VCT_SPEC_CASE(3) VCT_SPEC_CASE(4)
-            VCT_SPEC_CASE(5) VCT_SPEC_CASE(6) VCT_SPEC_CASE(7) VCT_SPEC_CASE(8)
-#undef VCT_SPEC_CASE
-        }
-    } else {
-        const dim3 grid((a.rays + 255) / 256, S, B);
-        const size_t lds = sizeof(float) * (size_t)NE * 9;
-        switch (M) {
-#define VCT_SPEC_CASE(MM) \
-    case MM: hipLaunchKernelGGL((k_batch_spectral<MM>), grid, dim3(256), lds, s, a); break;
-            VCT_SPEC_CASE(1) VCT_SPEC_CASE(2) VCT_SPEC_CASE(3) VCT_SPEC_CASE(4)
-            VCT_SPEC_CASE(5) VCT_SPEC_CASE(6) VCT_SPEC_CASE(7) VCT_SPEC_CASE(8)
-#undef VCT_SPEC_CASE
-        }
-    }
+    launch_batch_spectral(a, M, B, s);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }
@@ -2421,27 +2315,7 @@ vct_status vct_batch_spectral_groups(vct_plan* p, const float* const* d_L, const
     a.rays = p->g.n_views * p->g.n_channels; a.W = p->g.n_channels; a.VT = p->VT;
     a.B = B; a.S = S; a.M = M; a.NE = NE;
     hipLaunchKernelGGL(k_batch_stats_init, dim3((B * S + 63) / 64), dim3(64), 0, s, d_stats, B * S);
-    const size_t lds_all = sizeof(float) * (size_t)S * NE * 9 + sizeof(int) * kSpecAllWaves * S;
-    if (lds_all <= 64 * 1024) {
-        const dim3 grid((a.rays + kSpecAllBlock - 1) / kSpecAllBlock, 1, B);
-        switch (M) {
-#define VCT_SPEC_CASE(MM) \
-    case MM: hipLaunchKernelGGL((k_batch_spectral_all<MM>), grid, dim3(kSpecAllBlock), lds_all, s, a); break;
-            VCT_SPEC_CASE(1) VCT_SPEC_CASE(2) VCT_SPEC_CASE(3) VCT_SPEC_CASE(4)
-            VCT_SPEC_CASE(5) VCT_SPEC_CASE(6) VCT_SPEC_CASE(7) VCT_SPEC_CASE(8)
-#undef VCT_SPEC_CASE
-        }
-    } else {
-        const dim3 grid((a.rays + 255) / 256, S, B);
-        const size_t lds = sizeof(float) * (size_t)NE * 9;
-        switch (M) {
-#define VCT_SPEC_CASE(MM) \
-    case MM: hipLaunchKernelGGL((k_batch_spectral<MM>), grid, dim3(256), lds, s, a); break;
-            VCT_SPEC_CASE(1) VCT_SPEC_CASE(2) VCT_SPEC_CASE(3) VCT_SPEC_CASE(4)
-            VCT_SPEC_CASE(5) VCT_SPEC_CASE(6) VCT_SPEC_CASE(7) VCT_SPEC_CASE(8)
-#undef VCT_SPEC_CASE
-        }
-    }
+    launch_batch_spectral(a, M, B, s);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }

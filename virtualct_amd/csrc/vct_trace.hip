@@ -13,7 +13,8 @@
 //                per energy bin (M/main.cpp:492); here the trace is done once
 //                and the spectrum is applied afterwards.
 //   k_spectral   I_s = sum_E pdf_s(E) exp(-sum_m mu_s,m(E) L_m) with the
-//                spectrum tables of spectrum s in LDS, plus the per-spectrum
+//                spectrum tables of spectrum s in LDS (k_spectral_grad: with
+//                its derivatives in the L_m), plus the per-spectrum
 //                max/min used by the normalisation and the noise clamp.
 //   k_detector   max-normalisation + Gaussian noise (Philox4x32-10 +
 //                Box-Muller) + the reference's clamps.
@@ -29,6 +30,7 @@
 //                fixed point, one float atomic per voxel at the end.
 #include "vct_internal.h"
 #include "vct_march.h"
+#include "vct_spectral.h"
 
 #include <algorithm>
 #include <climits>
@@ -1351,16 +1353,58 @@ __global__ __launch_bounds__(kAdjBlock, 4) void k_trace_adj_tile(TraceArgs a, in
     }
 }
 
-// Polyenergetic sum: one spectrum per blockIdx.y; tables in LDS as
-// mu2[e][8] = -mu_m(E_e) * log2(e) and pdf[e].
-// Rays per workgroup of k_spectral: each workgroup adds its max and min of
-// I to the spectrum's two statistics words with one atomic each, and those
+// Polyenergetic sums.  Rays per workgroup: each workgroup adds its max and min
+// of I to the spectrum's two statistics words with one atomic each, and those
 // atomics serialise on the one address (1904 workgroups of 256 rays took as
-// long as the sums at 800 x 609), so workgroups are large.
+// long as the sums at 800 x 609), so workgroups are large, but for calls whose
+// large ones would leave CUs without any.
 constexpr int kSpecBlock = 1024;
 
-template <int M, bool DI>
+// Adds the workgroup's max and min of I (non-negative floats order like their
+// bits) to stats[0..1].  Every lane takes part.
+__device__ __forceinline__ void spec_stats(uint32_t* stats, bool valid, float I, uint32_t (&red)[2][kSpecBlock / 64])
+{
+    uint32_t mx = valid ? __float_as_uint(I) : 0u;
+    uint32_t mn = valid ? __float_as_uint(I) : 0x7f800000u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
+        mn = min(mn, (uint32_t)__shfl_xor((int)mn, off, 64));
+    }
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (lane == 0) { red[0][wave] = mx; red[1][wave] = mn; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int nw = (blockDim.x + 63) >> 6;
+        for (int w = 1; w < nw; w++) { mx = max(mx, red[0][w]); mn = min(mn, red[1][w]); }
+        atomicMax(stats, mx);
+        atomicMin(stats + 1, mn);
+    }
+}
+
+// The sums alone (spec_sum), one spectrum per blockIdx.y.
+template <int M>
 __global__ __launch_bounds__(kSpecBlock) void k_spectral(SpectralArgs a)
+{
+    extern __shared__ float lds[];
+    __shared__ uint32_t red[2][kSpecBlock / 64];
+    __shared__ int last[kSpecBlock / 64];
+    const int s = blockIdx.y, nr = a.V * a.W, traced = a.VT * a.W;
+    const SpecTable<M> tab =
+        SpecTable<M>::fill(lds, last, a.att + (size_t)s * M * a.NE, a.pdf + (size_t)s * a.NE, a.NE);
+    const int ray = blockIdx.x * blockDim.x + threadIdx.x, ray0 = ray & ~63;
+    SpecRays<M> L;
+    L.load([&](int t, int m) { return ray0 + t < traced ? a.L[(size_t)(ray0 + t) * 8 + m] : 0.f; });
+    float I = spec_sum<M>(tab, L);
+    if (ray >= traced) I = 0.f;
+    if (ray < nr) a.raw[(size_t)s * nr + ray] = I;
+    spec_stats(a.stats + 2 * s, ray < nr, I, red);
+}
+
+// The sums and their derivatives in the path integrals, one ray per lane; tables
+// in LDS as mu2[e][8] = -mu_m(E_e) * log2(e) and pdf[e].
+template <int M>
+__global__ __launch_bounds__(kSpecBlock) void k_spectral_grad(SpectralArgs a)
 {
     extern __shared__ float lds[];
     float* mu2 = lds;
@@ -1398,41 +1442,21 @@ __global__ __launch_bounds__(kSpecBlock) void k_spectral(SpectralArgs a)
             // hardware exp2: only terms below 2^-126 (flushed) differ from exp2f
             const float t = pdf[e] * __builtin_amdgcn_exp2f(x);
             I += t;
-            if (DI) {
 #pragma unroll
-                for (int m = 0; m < M; m++) d[m] = fmaf(t, mu[m], d[m]);
-            }
+            for (int m = 0; m < M; m++) d[m] = fmaf(t, mu[m], d[m]);
         }
     }
     if (valid) {
         a.raw[(size_t)s * nr + ray] = I;
-        if (DI) {
-            const float kLn2 = 0.69314718055994531f;
-            float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        const float kLn2 = 0.69314718055994531f;
+        float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int m = 0; m < M; m++) o[m] = d[m] * kLn2;
-            float4* dst = reinterpret_cast<float4*>(a.dIdL) + ((size_t)s * nr + ray) * 2;
-            dst[0] = make_float4(o[0], o[1], o[2], o[3]);
-            dst[1] = make_float4(o[4], o[5], o[6], o[7]);
-        }
+        for (int m = 0; m < M; m++) o[m] = d[m] * kLn2;
+        float4* dst = reinterpret_cast<float4*>(a.dIdL) + ((size_t)s * nr + ray) * 2;
+        dst[0] = make_float4(o[0], o[1], o[2], o[3]);
+        dst[1] = make_float4(o[4], o[5], o[6], o[7]);
     }
-    // block max / min of I (non-negative floats order like their bits)
-    uint32_t mx = valid ? __float_as_uint(I) : 0u;
-    uint32_t mn = valid ? __float_as_uint(I) : 0x7f800000u;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, off, 64));
-        mn = min(mn, (uint32_t)__shfl_xor((int)mn, off, 64));
-    }
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0) { red[0][wave] = mx; red[1][wave] = mn; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int nw = (blockDim.x + 63) >> 6;
-        for (int w = 1; w < nw; w++) { mx = max(mx, red[0][w]); mn = min(mn, red[1][w]); }
-        atomicMax(a.stats + 2 * s, mx);
-        atomicMin(a.stats + 2 * s + 1, mn);
-    }
+    spec_stats(a.stats + 2 * s, valid, I, red);
 }
 
 __global__ void k_stats_init(uint32_t* stats, int S)
@@ -1746,12 +1770,12 @@ template <int M>
 static void launch_spectral_m(const SpectralArgs& a, hipStream_t s)
 {
     const int nr = a.V * a.W;
-    const dim3 grid((nr + kSpecBlock - 1) / kSpecBlock, a.S);
-    const size_t lds = sizeof(float) * (size_t)a.NE * 9;
+    const int block = (long long)nr * a.S >= 128 * kSpecBlock ? kSpecBlock : 256;
+    const dim3 grid((nr + block - 1) / block, a.S);
     if (a.dIdL)
-        hipLaunchKernelGGL((k_spectral<M, true>), grid, dim3(kSpecBlock), lds, s, a);
+        hipLaunchKernelGGL((k_spectral_grad<M>), grid, dim3(block), sizeof(float) * (size_t)a.NE * 9, s, a);
     else
-        hipLaunchKernelGGL((k_spectral<M, false>), grid, dim3(kSpecBlock), lds, s, a);
+        hipLaunchKernelGGL((k_spectral<M>), grid, dim3(block), sizeof(float) * SpecTable<M>::floats(a.NE), s, a);
 }
 
 vct_status launch_spectral(const SpectralArgs& a, hipStream_t s)
