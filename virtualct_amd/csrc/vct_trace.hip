@@ -1717,13 +1717,12 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
         }
     } else if (adjoint) {
         if (a.VT > 0) {
-            // 2048 workgroups, four rounds of two per CU, and 4096 where their
-            // chunks keep eight views (380^2 x 722 views 1.16 -> 1.07 ms; 200^2 x
-            // 360, with four views each, 0.37 -> 0.41)
+            // at most 2048 workgroups, four full rounds of two per CU (380^2 x 722
+            // views 1.15 ms with the 2160 of 15 chunks, 1.13 with the 2016 of 14; 4096
+            // take 1.08, but a voxel's float adds and their rounding double)
             const int ntx = (a.N + kAdjTile - 1) / kAdjTile;
             const int ntiles = ntx * ntx;
-            const int target = (long long)ntiles * a.VT >= 8 * 4096 ? 4096 : 2048;
-            int nchunk = std::max(1, std::min(a.VT, (target + ntiles - 1) / ntiles));
+            int nchunk = std::max(1, std::min(a.VT, 2048 / ntiles));
             int cv = std::min((a.VT + nchunk - 1) / nchunk, kAdjMaxViews);
             if (a.adj_views > 0) cv = std::min(a.adj_views, kAdjMaxViews);
             nchunk = (a.VT + cv - 1) / cv;
