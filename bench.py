@@ -33,15 +33,13 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 MFMA_F32_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix
 SEGMENTS_512 = 282_824_404  # sum of per-ray segments at 512^2, 0.1 cm, 800x609
-# HBM bytes per tracer launch on this workload, from rocprofv3 --pmc passes
-# over `bench.py --steps 3 --warmup 1 --no-cpu-baseline --no-batched
-# --no-batch-fbp --copy-probe 256`: FETCH_SIZE 722793.1 KiB x 2.00 + WRITE_SIZE 15226.6 KiB
-# x 1.00, the factors being what the same counters read for the 256 MiB
-# device copy of the same run (131087.9 KiB fetched, 262144 KiB written).
-# The gathers read two 3.2 MB copies of the densities ([y][x] and [x][y]),
-# which overflow each XCD's 4 MB L2; the write is the 15.6 MB of path
-# integrals.
-TRACE_TRAFFIC_BYTES = int((722793.1 * 2.0 + 15226.6 * 1.0) * 1024)
+# HBM bytes per tracer launch on this workload, from rocprofv3 --pmc passes:
+# FETCH_SIZE 235700 KiB x 2.00 + WRITE_SIZE 15290 KiB x 1.00, the factors being
+# what the same counters read for a 256 MiB device copy (--copy-probe 256:
+# 131087.9 KiB fetched, 262144 KiB written).  The gathers read two 3.2 MB copies
+# of the densities ([y][x] and [x][y]), which overflow each XCD's 4 MB L2; the
+# write is the 15.6 MB of path integrals.
+TRACE_TRAFFIC_BYTES = int((235700 * 2.0 + 15290 * 1.0) * 1024)
 METRIC = "MBFPA ray·energy-bins/s, FBP voxel·views/s; batched grad steps/s vs plain"
 
 
@@ -431,7 +429,7 @@ def main():
         "mbfpa_ray_energy_bins_per_s": rays_bins / (mbfpa_ms * 1e-3),
         "fbp_voxel_views_per_s": p_mask * V / (fbp_ms * 1e-3),
         "roofline": {
-            "kernel": "k_trace_fwd_rot (tracer, quarter-turn orbits)",
+            "kernel": "k_trace_seg (tracer, quarter-turn orbits)",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
@@ -440,12 +438,12 @@ def main():
             "traffic": TRACE_TRAFFIC_BYTES,
             "algorithmic_bytes_per_launch": trace_bytes,
             "note": "algorithmic bytes = segments x 6 materials x 2 B (u16 densities) + V x W x 4 B; the "
-                    "traffic is what the L2s fetch and write (the two 3.2 MB density copies together exceed each "
-                    "XCD's 4 MB L2); the kernel is bound by its density gathers' texture path (TA / TD 84% / 90% "
-                    "busy) and FP64 VALU issue (49 VALU instructions per segment, 75% VALU busy)",
+                    "traffic is what the L2s fetch and write; the gathers are served by the caches, so the "
+                    "algorithmic rate can exceed the HBM peak, and the kernel is bound by FP64 VALU issue "
+                    "(28 VALU instructions per ray-segment, 83% VALU busy)",
         },
         "rooflines": [
-            {"kernel": "k_trace_fwd_rot (tracer, quarter-turn orbits)", "bound": "hbm", "unit": "GB/s", "achieved": achieved,
+            {"kernel": "k_trace_seg (tracer, quarter-turn orbits)", "bound": "hbm", "unit": "GB/s", "achieved": achieved,
              "peak": HBM_PEAK_GBS, "frac": achieved / HBM_PEAK_GBS,
              "per_launch": "segments x M x 2 B + V x W x 4 B"},
             {"kernel": "k_filter_prep + k_filter_gemm (filter stage)", "bound": "mfma", "unit": "TFLOP/s",
@@ -456,8 +454,8 @@ def main():
              "per_launch": "P_mask x V x 8 B + N^2 x 4 B = %.3f GB" % (bp_bytes / 1e9),
              "note": "the taps come from the 1.95 MB filtered sinogram held in L2 (16.6 MB of traffic "
                      "past the L2s per launch), so the algorithmic rate can exceed the HBM peak; the "
-                     "kernel is bound by VALU issue (76% busy, 17 VALU instructions per masked "
-                     "pixel-view) and the texture data path (75% busy)"},
+                     "kernel is bound by VALU issue (66% busy, 12 VALU instructions per masked "
+                     "pixel-view) and its gathers"},
         ],
         "cpu_baseline": None,
     }
