@@ -384,3 +384,49 @@ def test_tall_filter_products_equal_single_sinograms(gpu, W, V, S):
     many = ops.filter_sinogram(plan, p, 2).cpu().numpy()
     for i in (0, S // 2, S - 1):
         assert np.array_equal(many[i], ops.filter_sinogram(plan, p[i], 2)[0].cpu().numpy()), i
+
+
+@pytest.mark.parametrize("N,pix,V,S", [(512, 0.4, 8, 1), (512, 0.4, 6, 1), (512, 0.4, 5, 1), (512, 0.4, 8, 3),
+                                        (512, 0.4, 5, 13), (173, 1.0, 8, 1), (173, 1.0, 6, 1), (173, 1.0, 7, 2)])
+def test_pixels_level_with_the_source(gpu, N, pix, V, S):
+    """A field that holds the source's circle, with a line of pixels exactly at
+    the source's distance in view 0 (row 43 of 512 x 0.4 cm, row 1 of 173 x 1
+    cm: sid - Y = 0, and X = 0 too in the middle of the odd grid): they are off
+    the detector, as in the exact option.  Each term has five float roundings
+    and each image at most 8 adds, 13 * 2^-24 < 1e-6 of the summed magnitudes:
+    values up to 1.5 with weights up to 1.9 and 0.9, below 5 times a unit
+    sinogram's sum."""
+    import torch
+    from virtualct_amd import _lib
+    ops = _ops()
+    assert -(43 - 255.5) * 0.4 == 85.0 and -(1 - 86.0) * 1.0 == 85.0
+    plan, exact_plan = ops.Plan(_geom(N, pix, V)), _exact_plan(_geom(N, pix, V))
+    fl = _t(np.random.default_rng(N + V).uniform(0.5, 1.5, (S, V, 609)).astype(np.float32), gpu)
+    exact = ops.backproject(exact_plan, fl)
+    bound = 1e-6 * ops.backproject(exact_plan, torch.full_like(fl[:1], 5.0))
+    assert torch.isfinite(exact).all() and exact.count_nonzero() > 0
+    imgs = [ops.backproject(plan, fl)]
+    if S > 1:
+        imgs.append(torch.empty_like(imgs[0]))  # (the call without a workspace)
+        _lib.call("vct_backproject", plan.handle, fl.data_ptr(), S, imgs[1].data_ptr(),
+                  torch.cuda.current_stream().cuda_stream)
+    for img in imgs:
+        assert torch.isfinite(img).all()
+        assert torch.all((img - exact).abs() <= bound)
+    plan.close()
+    exact_plan.close()
+
+
+@pytest.mark.parametrize("S", [1, 2])
+def test_degenerate_channel_pitch(gpu, S):
+    """A channel pitch of zero puts every pixel off the detector, the middle
+    column (0 / 0) included, as in the exact option."""
+    import torch
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    fl = torch.ones((S, 8, 609), device=gpu)
+    for exact in (0, 1):
+        plan = ops.Plan(default_geometry(recon_size=65, pixel_cm=0.7, n_views=8, max_beta=0.0))
+        plan.set_option(_lib.OPT_EXACT_BACKPROJECT, exact)
+        assert not ops.backproject(plan, fl).any()
+        plan.close()

@@ -784,6 +784,7 @@ static BackprojArgs make_bp_args(const vct_plan* p, const float* d_fltd, float* 
     a.mask_r2 = a.mask_r * a.mask_r;
     a.exact = p->exact_bp;
     a.max_k = p->bp_max_k;
+    a.degenerate = !(std::isfinite(g.start_view_deg) && std::isfinite(g.sid_cm) && std::isfinite(a.inv_dbeta_ch));
     return a;
 }
 

@@ -264,11 +264,12 @@ static const double kAtanSym[kBpPoly] = {0.023298796324010433,  -0.0529659713247
                                          0.19999995815529828,   -0.3333333329437766,  0.9999999999993997};
 // Largest |tan(gamma)| of a masked pixel, the tangent from the source to the
 // mask circle of radius r (pixel centres lie within mask_r pitches), beyond
-// the polynomials' range.
+// the polynomials' range; also for a degenerate geometry, whose NaN channels
+// only the wide form tests for.
 static bool bp_wide(const BackprojArgs& a)
 {
     const double r = a.mask_r * a.pix;
-    return !(r < a.sid) || r / std::sqrt(a.sid * a.sid - r * r) > 0.49;
+    return a.degenerate || !(r < a.sid) || r / std::sqrt(a.sid * a.sid - r * r) > 0.49;
 }
 
 static void set_poly(BackprojArgs& a)
@@ -342,7 +343,10 @@ struct BpView {
 // terms differ from the exact ones by ~1e-7 relative.  Its geometry stays FP64
 // but takes fused multiply-adds where the exact form repeats the reference's
 // separate roundings, the source distance sid - Y in one pair of them, and the
-// bin without the range test of the cast (|gamma| < pi / 2 keeps it in range).
+// bin without the range test of the cast (|gamma| < pi / 2 keeps it in range;
+// WIDE fields hold pixels level with the source, where den = 0 makes tg NaN or
+// infinite: the library atan of X / den and the tested cast put them off the
+// detector as the exact form does, X = den = 0 included).
 // About 30 instead of 45 vector instructions per geometry, and per sinogram
 // three instead of four (a branch in place of a select): 512^2 x 800, one
 // sinogram in orbits 0.124 -> 0.106 ms, 12 per lane 1.12 -> 0.93 ms.
@@ -364,8 +368,8 @@ __device__ __forceinline__ BpView bp_view(const BackprojArgs& a, double xx, doub
 #pragma unroll
         for (int i = 1; i < kBpPoly; i++) p = __builtin_fma(p, u, a.poly[i]);
         double fGAM = __builtin_fma(tg, p, a.cent);
-        if (WIDE && fabs(tg) > 0.5) fGAM = __builtin_fma(atan(X / den), a.inv_dbeta_ch, a.cent);
-        const int GAM = (int)fGAM;
+        if (WIDE && !(fabs(tg) <= 0.5)) fGAM = __builtin_fma(atan(X / den), a.inv_dbeta_ch, a.cent);
+        const int GAM = WIDE ? trunc_i32_bp(fGAM) : (int)fGAM;
         const float w = (float)(fGAM - GAM);
         const float sf = __builtin_amdgcn_rcpf((float)L2) * (float)(a.dbeta_view * a.xfactor);
         g.w1s = w * sf;
@@ -733,8 +737,8 @@ __global__ __launch_bounds__(64 * kBpLoneWaves) void k_backproject_lone(Backproj
 #pragma unroll
             for (int i = 1; i < kBpLonePoly; i++) p = __builtin_fma(p, u, la.poly[i]);
             double fGAM = __builtin_fma(tg, p, (double)a.cent);
-            if (WIDE && fabs(tg) > 0.5) fGAM = __builtin_fma(atan(X / den), a.inv_dbeta_ch, (double)a.cent);
-            const int GAM = (int)fGAM;  // (|gamma| <= pi / 2 keeps it in range)
+            if (WIDE && !(fabs(tg) <= 0.5)) fGAM = __builtin_fma(atan(X / den), a.inv_dbeta_ch, (double)a.cent);
+            const int GAM = WIDE ? trunc_i32_bp(fGAM) : (int)fGAM;  // (as bp_view)
             const double s = rcp_f64(L2) * dbx;
             g.w1 = (fGAM - GAM) * s;
             g.w0 = s - g.w1;

@@ -115,6 +115,7 @@ struct BackprojArgs {
     int N, W, V, use_views, cent, half;
     int exact;            // 1: views in the reference's order per pixel, no 4-fold sharing
     int max_k;            // most sinograms per lane of the multi-sinogram kernel (0: kBpSinos)
+    int degenerate;       // an angle, the distance or the channel pitch is no finite number
     double pix, sid, dbeta_ch, inv_dbeta_ch, dbeta_view, xfactor, center, mask_r2, mask_r;
     double poly[kBpPoly] = {};  // channels per unit tan(gamma): the float-weight form's polynomial
 };
