@@ -377,3 +377,30 @@ def test_segment_tracer_equals_exact_march(gpu, N, fov, V, W, M, f32):
     np.testing.assert_array_equal(c, ce)
     assert np.isfinite(L).all() and not np.any(L[..., M:])
     assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9)
+
+
+@pytest.mark.parametrize("N,V,orbit", [(129, 80, 4), (128, 81, 4), (130, 22, 1)])
+def test_infinite_corner_voxel_reaches_its_own_rays_only(gpu, N, V, orbit):
+    """Float densities with +inf in voxel (0, 0), rays marched one by one by
+    segments (odd grid, odd view count, the orbit option): the rays past that
+    voxel are infinite, and all others keep their values, which the
+    exact-division march gives within two float roundings."""
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    geom = default_geometry(recon_size=N, pixel_cm=49.3 / N, n_views=V, n_channels=333, iso_channel=166.4)
+    d = np.random.default_rng(N).uniform(0.1, 2.0, (3, N, N)).astype(np.float32)
+    d[:, 0, 0] = np.inf
+    out = []
+    for exact in (0, 1):
+        plan = ops.Plan(geom)
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        plan.set_option(_lib.OPT_TRACE_ORBIT, orbit)
+        pk, dt = ops.pack_densities(plan, _t(d, gpu))
+        out.append(ops.trace_paths(plan, pk, dt, 3).cpu().numpy())
+        plan.close()
+    L, Le = out
+    far = np.isfinite(Le)
+    assert 0 < np.count_nonzero(~far) < Le.size // 4
+    np.testing.assert_array_equal(L[~far], Le[~far])
+    assert np.isfinite(L[far]).all()
+    assert np.all(np.abs(L[far] - Le[far]) <= 2.0 ** -22 * np.abs(Le[far]) + 1e-9)

@@ -1030,7 +1030,10 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
                     i++;
                     return end;
                 };
+                // (outside the image a lone ray holds voxel 0 with length 0, which an
+                // infinite density would turn into NaN; an orbit reads the zero border)
                 auto add = [&](const Pending& p) {
+                    if (R == 1 && DT == VCT_DENS_F32 && p.rr == 0.0) return;
 #pragma unroll
                     for (int k = 0; k < R; k++) sums.add(k, p.q[k], p.rr);
                 };
