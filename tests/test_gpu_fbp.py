@@ -430,3 +430,30 @@ def test_degenerate_channel_pitch(gpu, S):
         plan.set_option(_lib.OPT_EXACT_BACKPROJECT, exact)
         assert not ops.backproject(plan, fl).any()
         plan.close()
+
+
+@pytest.mark.parametrize("S", [1, 4])
+def test_float_weights_near_a_channel(gpu, oracle, S):
+    """Every third channel of one view is 1, so a pixel's value is one
+    interpolation weight over L^2.  Both weights keep 24 bits where they are
+    small: at most seven roundings of 2^-24 (L^2, its reciprocal (two), the view
+    step, their product, the weight and its product) and 2e-10 channels of the
+    arc tangent over the weight, together below 6e-7 for weights from 2e-3 on.
+    (A float 1 - w made from a float w is off by 1.5e-5 there.)"""
+    ops = _ops()
+    N, pix, V, view = 256, 0.2, 16, 3
+    plan = ops.Plan(_geom(N, pix, V))
+    fl = np.zeros((V, 609), np.float32)
+    fl[view, ::3] = 1.0
+    ones = np.zeros((V, 609))
+    ones[view] = 1.0
+    g = Geom(N=N, pix=pix, V=V)
+    f64 = oracle.backproject_f64(g, fl.astype(np.float64))
+    whole = oracle.backproject_f64(g, ones)
+    img = ops.backproject(plan, _t(np.repeat(fl[None], S, 0), gpu)).cpu().numpy().astype(np.float64)
+    weight = np.divide(f64, whole, out=np.zeros_like(f64), where=whole != 0)
+    use = weight >= 2e-3
+    assert np.count_nonzero(use & (weight < 2e-2)) > 100
+    for k in range(S):
+        assert np.all(np.abs(img[k] - f64)[use] <= 6e-7 * np.abs(f64[use]))
+    plan.close()

@@ -370,10 +370,11 @@ __device__ __forceinline__ BpView bp_view(const BackprojArgs& a, double xx, doub
         double fGAM = __builtin_fma(tg, p, a.cent);
         if (WIDE && !(fabs(tg) <= 0.5)) fGAM = __builtin_fma(atan(X / den), a.inv_dbeta_ch, a.cent);
         const int GAM = WIDE ? trunc_i32_bp(fGAM) : (int)fGAM;
-        const float w = (float)(fGAM - GAM);
+        // (1 - w in FP64: both weights keep 24 bits where they are small)
+        const double w = fGAM - GAM;
         const float sf = __builtin_amdgcn_rcpf((float)L2) * (float)(a.dbeta_view * a.xfactor);
-        g.w1s = w * sf;
-        g.w0s = fmaf(-w, sf, sf);
+        g.w1s = (float)w * sf;
+        g.w0s = (float)(1.0 - w) * sf;
         g.ok = (unsigned)GAM < (unsigned)(a.W - 1);
         g.col = g.ok ? GAM : 0;
     } else {
