@@ -327,3 +327,32 @@ def test_tile_adjoint_segments_equal_the_exact_march(gpu, N, pix, V, M, views):
         plan.close()
     assert rel_max(out[0], out[1]) < 1e-6
     assert np.count_nonzero(out[1][..., :M]) > 0 and np.all(out[0][..., M:] == 0)
+
+
+def test_wide_detectors_keep_the_sums_scale(gpu):
+    """8192 channels x 256 views, more than 2^19 rays over one tile: the
+    fixed-point scale is that of a few views per workgroup.  The largest weight
+    of every 16 views sits on a ray just outside the image; the others are
+    2^-28 of it, so their products with the segments are about one unit of the
+    scale and a coarser one would lose them.  The sums are exact integers, so
+    chunks of 16 and of up to 256 views differ by float adds only (16 * 2^-24)."""
+    import torch
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    N, V, W = 32, 256, 8192
+    plan = ops.Plan(default_geometry(recon_size=N, pixel_cm=0.6, n_views=V, n_channels=W, iso_channel=W / 2.0))
+    pk, dt = ops.pack_densities(plan, torch.ones((1, N, N), device=gpu))
+    hit = ops.trace_paths(plan, pk, dt, 1)[..., 0] > 0
+    last = (hit * torch.arange(W, device=gpu)).amax(1)  # the last channel that meets the image
+    assert int(hit.sum()) > 1 << 19 and int(last.max()) + 40 < W
+    w = torch.zeros((V, W, 8), device=gpu)
+    w[..., 0] = 2.0 ** -28
+    w[torch.arange(V, device=gpu), last + 40, 0] = 1.0
+    grads = []
+    for views in (16, 256):
+        plan.set_option(_lib.OPT_ADJOINT_VIEWS, views)
+        grads.append(ops.trace_adjoint(plan, w, 1)[..., 0].cpu().numpy().astype(np.float64))
+    few, many = grads
+    assert few.min() > 0 and few.max() < 1e-2
+    assert np.all(np.abs(many - few) <= 1e-6 * few)
+    plan.close()

@@ -397,13 +397,18 @@ struct SinkRot {
 // meet a column of the tile at one step when x is the major axis).  FIXED:
 // the accumulator is 51-bit fixed point, each contribution rounded to an
 // integer after scaling by a power of two that keeps it below 2^30 in
-// magnitude (and 2^19 of them in range); the sums are then exact (and
-// independent of the order of the adds), and ds_add_u64 runs about ten times faster than ds_add_f32 on
-// gfx950 (0.3 vs 3.4 lane-operations per clock per CU, measured).  The float
+// magnitude; the sums of up to kAdjMaxRays rays are then exact (and
+// independent of the order of the adds), and ds_add_u64 runs about ten times
+// faster than ds_add_f32 on gfx950 (0.3 vs 3.4 lane-operations per clock per
+// CU, measured).  The float
 // form serves workgroups whose weights are not all finite, so NaN and
 // infinity reach the gradient as with float sums.
 constexpr int kAdjTile = 32;
 constexpr int kAdjMaxViews = 256;  // views per workgroup
+// Rays per workgroup: what 2^19 rays add to a voxel at the full scale stays
+// within the sums' 51 bits (a ray at most sqrt(2) 2^30: its first segment and
+// its others there).  8192 channels take at most 64 views.
+constexpr int kAdjMaxRays = 1 << 19;
 constexpr int kAdjBlock = 512;
 
 template <int M, bool FIXED>
@@ -1295,8 +1300,7 @@ __global__ __launch_bounds__(kAdjBlock, 4) void k_trace_adj_tile(TraceArgs a, in
     if (fixed) {
         int e;
         frexpf(wl, &e);  // wl < 2^e, e >= -79
-        // (2^19 rays' contributions stay within the sums' 51 bits)
-        S = 30 - e - max(0, 32 - __clz(total) - 19);  // <= 109
+        S = 30 - e;      // <= 109
     }
     const double scale = ldexp(1.0, S);
     bool ovf = false;
@@ -1728,6 +1732,7 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
             int nchunk = std::max(1, std::min(a.VT, 2048 / ntiles));
             int cv = std::min((a.VT + nchunk - 1) / nchunk, kAdjMaxViews);
             if (a.adj_views > 0) cv = std::min(a.adj_views, kAdjMaxViews);
+            cv = std::max(1, std::min(cv, kAdjMaxRays / a.W));
             nchunk = (a.VT + cv - 1) / cv;
             const int per_xcd = (ntiles * nchunk + 7) / 8;
             hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, cv,
