@@ -150,9 +150,10 @@ vct_status vct_plan_destroy(vct_plan* plan);
  * VCT_OPT_BP_SINOS_PER_LANE = 7: most sinograms one lane backprojects in a
  * multi-sinogram call, 2..16 (0: 16); images are bit-identical for every value.
  * VCT_OPT_ADJOINT_VIEWS = 8: most views per workgroup of the adjoint, 1..256
- * and no more than 2^19 / n_channels (0: a chunk that gives at most 2048
- * workgroups); workgroups of other chunks add
- * their tiles in another order, which changes the float rounding of grad. */
+ * and no more than 2^19 / n_channels (0: even chunks that give at most 2048
+ * workgroups, or more where a chunk would exceed those views); workgroups of
+ * other chunks add their tiles in another order, which changes the float
+ * rounding of grad. */
 enum {
     VCT_OPT_EXACT_TRACE = 1,
     VCT_OPT_MAX_STEPS = 2,

@@ -183,3 +183,42 @@ def test_tuner_keeps_the_fastest_and_caches_it(tmp_path):
     assert t.best(("ramp",), lambda: [{"x": 1}, {"x": 2}], ramp) == {"x": 1}
     assert Tuner(path).best(("k", 1), lambda: [{"x": 1}], time_fn) == {"x": 2}
     assert t.best(("k", 2), lambda: [{"x": 3}, {"x": 1}], time_fn) == {"x": 3}
+
+
+@pytest.fixture(scope="module")
+def split(tmp_path_factory):
+    """The launch rules of csrc/vct_split.h as a host library."""
+    import subprocess
+    d = tmp_path_factory.mktemp("split")
+    src, lib = d / "split.cpp", d / "libsplit.so"
+    src.write_text('#include "vct_split.h"\n'
+                   'extern "C" void adjoint_split(int t, int v, int w, int a, int* o)\n'
+                   '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "virtualct_amd", "csrc"),
+                    str(src), "-o", str(lib)], check=True, capture_output=True)
+    return C.CDLL(str(lib))
+
+
+def test_adjoint_chunks_are_even_and_bounded(split):
+    """Chunks of the tile adjoint: every view in one, at most 256 views and 2^19
+    rays, as even as they go, and at most 2048 workgroups unless those bounds
+    ask for more (768^2 x 800 views: four chunks of 200, not 256, 256, 256, 32)."""
+    out = (C.c_int * 2)()
+
+    def of(ntiles, views, channels, asked=0):
+        split.adjoint_split(ntiles, views, channels, asked, out)
+        return out[0], out[1]
+    assert of(576, 800, 609) == (200, 4) and of(144, 722, 609) == (52, 14) and of(1024, 256, 8192) == (64, 4)
+    for channels in (22, 609, 2048, 2049, 8192):
+        most = min(256, (1 << 19) // channels)
+        for n in (1, 2, 3, 12, 23, 24, 32, 45, 46, 64, 256):
+            for views in (2, 3, 5, 161, 255, 256, 257, 722, 800, 2100, 65536):
+                per, chunks = of(n * n, views, channels)
+                assert 1 <= per <= most and (chunks - 1) * per < views <= chunks * per
+                least = -(-views // most)
+                assert n * n * chunks <= 2048 or chunks == least or n * n > 2048 and chunks == max(1, least)
+                # no split into as many chunks has a smaller largest one
+                assert per == -(-views // chunks)
+                for asked in (1, 7, 256):
+                    p, c = of(n * n, views, channels, asked)
+                    assert p == min(asked, most) and (c - 1) * p < views <= c * p

@@ -31,6 +31,7 @@
 #include "vct_internal.h"
 #include "vct_march.h"
 #include "vct_spectral.h"
+#include "vct_split.h"
 
 #include <algorithm>
 #include <climits>
@@ -404,11 +405,6 @@ struct SinkRot {
 // form serves workgroups whose weights are not all finite, so NaN and
 // infinity reach the gradient as with float sums.
 constexpr int kAdjTile = 32;
-constexpr int kAdjMaxViews = 256;  // views per workgroup
-// Rays per workgroup: what 2^19 rays add to a voxel at the full scale stays
-// within the sums' 51 bits (a ray at most sqrt(2) 2^30: its first segment and
-// its others there).  8192 channels take at most 64 views.
-constexpr int kAdjMaxRays = 1 << 19;
 constexpr int kAdjBlock = 512;
 
 template <int M, bool FIXED>
@@ -1724,18 +1720,10 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
         }
     } else if (adjoint) {
         if (a.VT > 0) {
-            // at most 2048 workgroups, four full rounds of two per CU (380^2 x 722
-            // views 1.15 ms with the 2160 of 15 chunks, 1.13 with the 2016 of 14; 4096
-            // take 1.08, but a voxel's float adds and their rounding double)
-            const int ntx = (a.N + kAdjTile - 1) / kAdjTile;
-            const int ntiles = ntx * ntx;
-            int nchunk = std::max(1, std::min(a.VT, 2048 / ntiles));
-            int cv = std::min((a.VT + nchunk - 1) / nchunk, kAdjMaxViews);
-            if (a.adj_views > 0) cv = std::min(a.adj_views, kAdjMaxViews);
-            cv = std::max(1, std::min(cv, kAdjMaxRays / a.W));
-            nchunk = (a.VT + cv - 1) / cv;
-            const int per_xcd = (ntiles * nchunk + 7) / 8;
-            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, cv,
+            const int ntx = (a.N + kAdjTile - 1) / kAdjTile, ntiles = ntx * ntx;
+            const AdjointSplit sp = adjoint_split(ntiles, a.VT, a.W, a.adj_views);
+            const int per_xcd = (ntiles * sp.chunks + 7) / 8;
+            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, sp.views,
                                per_xcd, seg_planes(a) ? 1 : 0);
         }
     } else if (!a.exact && a.n_rays <= INT_MAX / 8) {
