@@ -457,3 +457,34 @@ def test_float_weights_near_a_channel(gpu, oracle, S):
     for k in range(S):
         assert np.all(np.abs(img[k] - f64)[use] <= 6e-7 * np.abs(f64[use]))
     plan.close()
+
+
+def test_backprojection_workspace_serves_smaller_calls(gpu):
+    """A workspace sized for a count of sinograms serves every smaller count
+    and every VCT_OPT_BP_SINOS_PER_LANE: the size grows with the count and does
+    not depend on the option, and no call writes past it."""
+    import torch
+    from virtualct_amd import _lib
+    ops = _ops()
+    N, pix, V = 512, 0.1, 8
+    plan = ops.Plan(_geom(N, pix, V))
+    size = lambda n: int(_lib.lib().vct_backproject_workspace_bytes(plan.handle, n))
+    sizes = []
+    for cap in (0, 2, 3, 4, 6, 8, 11, 16):
+        plan.set_option(_lib.OPT_BP_SINOS_PER_LANE, cap)
+        sizes.append([size(n) for n in range(1, 70)])
+    assert all(s == sizes[0] for s in sizes)
+    assert sizes[0] == sorted(sizes[0]) and sizes[0][0] == 0 and sizes[0][1] > 0
+    slot = V * 609
+    fl = torch.randn((50, V, 609), device=gpu)
+    for most in (3, 13, 25, 50):
+        words = size(most) // 4
+        buf = torch.full((48 * slot + words,), 7.0, device=gpu)  # (more than any call can use)
+        for n in sorted({2, most - 2, most - 1, most, most * 24 // 25} - {1}):
+            for cap in (0, 4, 8):
+                plan.set_option(_lib.OPT_BP_SINOS_PER_LANE, cap)
+                img = torch.empty((n, N, N), device=gpu)
+                _lib.call("vct_backproject_ws", plan.handle, fl.data_ptr(), n, img.data_ptr(), buf.data_ptr(),
+                          torch.cuda.current_stream().cuda_stream)
+                assert torch.all(buf[words:] == 7.0), (most, n, cap)
+    plan.close()

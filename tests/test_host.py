@@ -193,7 +193,10 @@ def split(tmp_path_factory):
     src, lib = d / "split.cpp", d / "libsplit.so"
     src.write_text('#include "vct_split.h"\n'
                    'extern "C" void adjoint_split(int t, int v, int w, int a, int* o)\n'
-                   '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n')
+                   '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n'
+                   'extern "C" int il_slots(int N, int cap, int S)\n'
+                   '{ int K = vct::bp_interleave_width(N, false, cap, S); return K ? vct::bp_interleave_slots(S, K) : 0; }\n'
+                   'extern "C" int il_bound(int S) { return vct::bp_interleave_bound(S); }\n')
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "virtualct_amd", "csrc"),
                     str(src), "-o", str(lib)], check=True, capture_output=True)
     return C.CDLL(str(lib))
@@ -222,3 +225,16 @@ def test_adjoint_chunks_are_even_and_bounded(split):
                 for asked in (1, 7, 256):
                     p, c = of(n * n, views, channels, asked)
                     assert p == min(asked, most) and (c - 1) * p < views <= c * p
+
+
+def test_interleave_bound_covers_every_smaller_call(split):
+    """The workspace of several interleaved sinograms, sized for a count, serves
+    every smaller count at every image size and option (50 sinograms at 512^2
+    use 40 slots, 48 use 48), and stays within one pass."""
+    bounds = [split.il_bound(n) for n in range(0, 60)]
+    assert bounds[:3] == [0, 0, 2] and bounds == sorted(bounds) and bounds[-1] == bounds[48] == 48
+    assert split.il_slots(512, 0, 50) == 40 and split.il_slots(512, 0, 48) == 48
+    for N in (2, 64, 97, 128, 200, 300, 512, 8192):
+        for cap in (0, *range(2, 17)):
+            for n in (*range(1, 100), 65535):
+                assert split.il_slots(N, cap, n) <= bounds[min(n, 59)], (N, cap, n)

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "vct_internal.h"
+#include "vct_split.h"
 
 // Work buffer of vct_mbfpa_forward_noalloc (path integrals, raw sums and
 // their statistics), one copy per GPU, held until the process ends.  Host
@@ -796,17 +797,10 @@ vct_status vct_backproject(vct_plan* p, const float* d_fltd, int n_sino, float* 
     return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, pick_stream(p, stream));
 }
 
-// Sinograms that one pass of vct_backproject_ws interleaves (a bound on its
-// workspace).
-constexpr int kIlPass = 48;
-
 size_t vct_backproject_workspace_bytes(const vct_plan* p, int n_sino)
 {
     if (!p || n_sino < 1) return 0;
-    const int K = bp_interleave_width(make_bp_args(p, nullptr, nullptr), n_sino);
-    if (K == 0) return 0;
-    const int n = std::min(n_sino, kIlPass / K * K);
-    return (size_t)((n + K - 1) / K) * K * p->g.n_views * p->g.n_channels * sizeof(float);
+    return (size_t)bp_interleave_bound(std::min(n_sino, kIlPass)) * p->g.n_views * p->g.n_channels * sizeof(float);
 }
 
 vct_status vct_backproject_ws(vct_plan* p, const float* d_fltd, int n_sino, float* d_img, void* d_work, void* stream)
@@ -815,11 +809,11 @@ vct_status vct_backproject_ws(vct_plan* p, const float* d_fltd, int n_sino, floa
     if (!p || !d_fltd || !d_img) return set_error(VCT_ERR_ARG, "NULL argument");
     if (n_sino < 1 || n_sino > 65535) return set_error(VCT_ERR_ARG, "n_sino %d invalid", n_sino);
     hipStream_t s = pick_stream(p, stream);
-    const int K = d_work ? bp_interleave_width(make_bp_args(p, nullptr, nullptr), n_sino) : 0;
+    const int K = d_work ? bp_interleave_width(p->g.recon_size, p->exact_bp != 0, p->bp_max_k, n_sino) : 0;
     if (K == 0) return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, s);
     const int VW = p->g.n_views * p->g.n_channels;
     const size_t NN = (size_t)p->g.recon_size * p->g.recon_size;
-    const int pass = kIlPass / K * K;
+    const int pass = bp_interleave_pass(K);
     for (int i = 0; i < n_sino; i += pass) {
         const int n = std::min(n_sino - i, pass);
         VCT_CHECK(launch_interleave_sinos(d_fltd + (size_t)i * VW, n, VW, K, (float*)d_work, s));

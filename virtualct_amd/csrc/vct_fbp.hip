@@ -931,23 +931,6 @@ vct_status launch_interleave_sinos(const float* src, int S, int VW, int K, float
     return VCT_OK;
 }
 
-// Width of the interleaved slices that S sinograms take, 0 for none (a single
-// sinogram, the exact option).  The fewest slices of at most 12, but enough
-// that the launch has kBpIlLanes lanes, and then the narrowest width that
-// holds an even share.  Measured (us, one launch, 800 views): 16 sinograms at
-// 512^2 as 3 x 6, 2 x 8, 12 + 4 and 1 x 16 867, 889, 1103 and 1235; 12 at
-// 300^2 as 2 x 6, 12 and 3 x 4 291, 319 and 363; 12 at 200^2 x 360 views as
-// 3 x 4, 2 x 6, 12 and 6 x 2 104, 114, 117 and 148.
-int bp_interleave_width(const BackprojArgs& a, int S)
-{
-    constexpr long long kBpIlLanes = 1 << 17;
-    if (S < 2 || a.exact) return 0;
-    const long long px = (long long)a.N * a.N;
-    const int cap = a.max_k >= 2 && a.max_k < 12 ? a.max_k / 2 * 2 : 12;
-    const int slices = std::max((S + cap - 1) / cap, (int)std::min<long long>((S + 1) / 2, (kBpIlLanes + px - 1) / px));
-    return ((S + slices - 1) / slices + 1) / 2 * 2;
-}
-
 vct_status launch_backproject_il(const BackprojArgs& args, int S, int K, hipStream_t s)
 {
     BackprojArgs a = args;

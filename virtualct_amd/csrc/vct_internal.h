@@ -204,7 +204,6 @@ vct_status launch_filter(const FilterPrepArgs& p, const FilterGemmArgs& g, hipSt
 vct_status launch_backproject(const BackprojArgs& a, int S, hipStream_t s);
 // S sinograms interleaved in slices of K (bp_interleave_width)
 vct_status launch_backproject_il(const BackprojArgs& a, int S, int K, hipStream_t s);
-int bp_interleave_width(const BackprojArgs& a, int S);
 // il: every group's sinograms interleaved in slices of K (4, 8, 12 or 16)
 vct_status launch_backproject_groups(BpGroups& ga, int K, hipStream_t s, bool il = false);
 vct_status launch_interleave_sinos(const float* src, int S, int VW, int K, float* dst, hipStream_t s);

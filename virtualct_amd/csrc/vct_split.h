@@ -35,4 +35,42 @@ inline AdjointSplit adjoint_split(int ntiles, int views, int channels, int asked
     return {per, chunks_of(per)};
 }
 
+// ------------------------------ several sinograms per call (vct_backproject_ws)
+
+constexpr int kIlWidth = 12;  // widest slice
+constexpr int kIlPass = 48;   // most sinograms that one pass interleaves (bounds the workspace)
+
+// Width of the interleaved slices that S sinograms of N^2 pixels take, 0 for
+// none (a single sinogram, the exact option).  The fewest slices of at most
+// kIlWidth (max_k: VCT_OPT_BP_SINOS_PER_LANE), but enough that the launch has
+// kIlLanes lanes, and then the narrowest width that holds an even share.
+// Measured (us, one launch, 800 views): 16 sinograms at 512^2 as 3 x 6, 2 x 8,
+// 12 + 4 and 1 x 16 867, 889, 1103 and 1235; 12 at 300^2 as 2 x 6, 12 and 3 x 4
+// 291, 319 and 363; 12 at 200^2 x 360 views as 3 x 4, 2 x 6, 12 and 6 x 2 104,
+// 114, 117 and 148.
+inline int bp_interleave_width(int N, bool exact, int max_k, int S)
+{
+    constexpr long long kIlLanes = 1 << 17;
+    if (S < 2 || exact) return 0;
+    const long long px = (long long)N * N;
+    const int cap = max_k >= 2 && max_k < kIlWidth ? max_k / 2 * 2 : kIlWidth;
+    const int slices = std::max((S + cap - 1) / cap, (int)std::min<long long>((S + 1) / 2, (kIlLanes + px - 1) / px));
+    return ((S + slices - 1) / slices + 1) / 2 * 2;
+}
+
+// Sinograms per pass of slices of K, and the slots that S of them take.
+inline int bp_interleave_pass(int K) { return kIlPass / K * K; }
+inline int bp_interleave_slots(int S, int K) { return std::min((S + K - 1) / K * K, bp_interleave_pass(K)); }
+
+// Slots that serve up to S sinograms at any width that such a call can take,
+// whatever the options: it grows with S, so a workspace sized for the largest
+// call serves the others.
+inline int bp_interleave_bound(int S)
+{
+    int slots = 0;
+    for (int K = 2; K <= std::min(kIlWidth, (S + 1) / 2 * 2); K += 2)
+        if (S >= 2) slots = std::max(slots, bp_interleave_slots(S, K));
+    return slots;
+}
+
 }  // namespace vct
