@@ -404,3 +404,68 @@ def test_infinite_corner_voxel_reaches_its_own_rays_only(gpu, N, V, orbit):
     np.testing.assert_array_equal(L[~far], Le[~far])
     assert np.isfinite(L[far]).all()
     assert np.all(np.abs(L[far] - Le[far]) <= 2.0 ** -22 * np.abs(Le[far]) + 1e-9)
+
+
+@pytest.mark.parametrize("N,fov,V,W,M,f32", [
+    (128, 51.2, 48, 333, 6, False), (128, 51.2, 48, 333, 5, False), (128, 51.2, 50, 333, 8, False),
+    (384, 51.2, 12, 609, 8, False), (384, 51.2, 14, 333, 6, True), (300, 48.0, 12, 333, 8, True),
+    (384, 51.2, 13, 333, 6, False), (65, 26.0, 20, 333, 8, True)])
+def test_stepwise_tracers_equal_exact_march(gpu, N, fov, V, W, M, f32):
+    """Grids whose plane middles meet grid lines keep the marches that go step
+    by step (orbits of 4 and 2 rays, odd view counts and odd grids ray by ray):
+    the same counters as the exact-division march, path integrals within two
+    float roundings, and the same bits for every workgroup size."""
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    D = fov / N
+    middles = np.arange(int(N // 2 * D) + 3) / D + 0.5
+    assert np.abs(middles - np.rint(middles)).min() < 1e-6
+    geom = default_geometry(recon_size=N, pixel_cm=D, n_views=V, n_channels=W, iso_channel=W / 2.0 + 0.13)
+    rng = np.random.default_rng(N + V)
+    if f32:
+        d = rng.uniform(0.0, 2.0, (M, N, N)).astype(np.float32)
+        d[:, N // 2, 1] = -1.0
+    else:
+        d = rng.integers(0, 2000, (M, N, N)).astype(np.int16)
+    out = []
+    for exact, block in ((1, 0), (0, 64), (0, 128), (0, 256)):
+        plan = ops.Plan(geom)
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        plan.set_option(_lib.OPT_TRACE_BLOCK, block)
+        pk, dt = ops.pack_densities(plan, _t(d, gpu))
+        L, cnt = ops.trace_paths(plan, pk, dt, M, counts=True)
+        out.append((L.cpu().numpy(), cnt.cpu().numpy()))
+        plan.close()
+    (Le, ce), (L, c) = out[0], out[1]
+    assert ce.sum() > 0
+    np.testing.assert_array_equal(c, ce)
+    assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9)
+    for Lb, cb in out[2:]:
+        assert np.array_equal(Lb, L) and np.array_equal(cb, c)
+
+
+@pytest.mark.parametrize("N,V,M,f32,orbit", [(129, 20, 6, False, 4), (129, 22, 8, True, 4), (128, 21, 6, False, 4),
+                                              (128, 23, 3, True, 4), (130, 20, 8, False, 1), (130, 20, 7, True, 1)])
+def test_lone_ray_segments_equal_exact_march(gpu, N, V, M, f32, orbit):
+    """One ray per march by segments (odd grids and view counts, the orbit
+    option), on grids without plane middles on grid lines: counters and path
+    integrals as above."""
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    geom = default_geometry(recon_size=N, pixel_cm=49.3 / N, n_views=V, n_channels=333, iso_channel=166.63)
+    rng = np.random.default_rng(N + V)
+    d = rng.uniform(0.0, 2.0, (M, N, N)).astype(np.float32) if f32 else \
+        rng.integers(0, 2000, (M, N, N)).astype(np.int16)
+    out = []
+    for exact in (0, 1):
+        plan = ops.Plan(geom)
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        plan.set_option(_lib.OPT_TRACE_ORBIT, orbit)
+        pk, dt = ops.pack_densities(plan, _t(d, gpu))
+        L, cnt = ops.trace_paths(plan, pk, dt, M, counts=True)
+        out.append((L.cpu().numpy(), cnt.cpu().numpy()))
+        plan.close()
+    (L, c), (Le, ce) = out
+    assert ce.sum() > 0
+    np.testing.assert_array_equal(c, ce)
+    assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9)
