@@ -148,7 +148,8 @@ vct_status vct_plan_destroy(vct_plan* plan);
  * the tracers that march step by step (the exact option, the r >= rmax test,
  * grids whose plane middles fall on grid lines); the others use 512.
  * VCT_OPT_BP_SINOS_PER_LANE = 7: most sinograms one lane backprojects in a
- * multi-sinogram call, 2..16 (0: 16); images are bit-identical for every value.
+ * multi-sinogram call, 2..16 (0: 16, and never more than 12 in
+ * vct_backproject_ws); images are bit-identical for every value.
  * VCT_OPT_ADJOINT_VIEWS = 8: most views per workgroup of the adjoint, 1..256
  * and no more than 2^19 / n_channels (0: even chunks that give at most 2048
  * workgroups, or more where a chunk would exceed those views); workgroups of
@@ -164,6 +165,9 @@ enum {
     VCT_OPT_ADJOINT_VIEWS = 8
 };
 vct_status vct_plan_set_option(vct_plan* plan, int option, int value);
+/* 1 if a vct_trace_paths call of the plan with these densities marches step by
+ * step, so that VCT_OPT_TRACE_BLOCK sets its workgroups, else 0. */
+int vct_plan_uses_trace_block(const vct_plan* plan, int dens_type, int M);
 
 /* ------------------------------------------------------- host-side tables */
 

@@ -109,3 +109,18 @@ def test_batch_forward_fbp_consults_the_tuner(gpu, tmp_path, monkeypatch):
     s2, i2 = fixed.run()
     for a, b in zip(s1 + i1, s2 + i2):
         assert rel_max(a.cpu().numpy(), b.cpu().numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("N,pix,blocks", [(128, 0.35, 1), (128, 0.4, 3)])
+def test_tuner_times_only_shapes_that_differ(gpu, tmp_path, monkeypatch, N, pix, blocks):
+    """The segment tracer has one workgroup size, so on its grids there is one
+    candidate; 128 x 0.4 cm marches step by step and has three.  Caps of more
+    than 12 sinograms per lane are the same call as 12."""
+    from virtualct_amd import autotune, ops
+    monkeypatch.setattr(autotune, "_tuner", autotune.Tuner(str(tmp_path / "tune.json")))
+    plan = ops.Plan(_geom(N, pix, 160))
+    plan.tune(6, n_sino=16, what=("trace", "backproject"))
+    timed = {e["key"][0]: [cfg for _, cfg in e["results"]] for e in autotune.tuner().log}
+    assert len(timed["trace block"]) == blocks
+    assert max(c["bp_sinos_per_lane"] for c in timed["bp sinograms per lane"]) <= 12
+    plan.close()

@@ -72,6 +72,7 @@ _SIGS = {
     "vct_plan_create": (C.c_int, [_P, C.POINTER(Geometry), C.POINTER(_P)]),
     "vct_plan_destroy": (C.c_int, [_P]),
     "vct_plan_set_option": (C.c_int, [_P, C.c_int, C.c_int]),
+    "vct_plan_uses_trace_block": (C.c_int, [_P, C.c_int, C.c_int]),
     "vct_attenuation_coefficient": (C.c_int, [C.c_char_p, C.c_int, _P, _P, C.c_int, _P, _P,
                                                C.POINTER(C.c_int), _P]),
     "vct_const_map": (C.c_int, [C.POINTER(Geometry), C.c_int, _P]),

@@ -96,7 +96,7 @@ def events_ms(fn, reps: int = 3) -> float:
 
 TRACE_BLOCKS = (64, 128, 256)
 ADJOINT_VIEWS = (0, 25, 50, 100, 200)
-BP_SINOS_PER_LANE = (4, 8, 12, 16)
+BP_SINOS_PER_LANE = (4, 8, 12)  # (ops.backproject takes 12 at most)
 
 
 def tune_plan(plan, M: int = 6, n_sino: int = 1, what=("trace", "adjoint", "backproject")) -> dict:
@@ -119,7 +119,9 @@ def tune_plan(plan, M: int = 6, n_sino: int = 1, what=("trace", "adjoint", "back
         def t_trace(cfg):
             plan.set_option(_lib.OPT_TRACE_BLOCK, cfg["trace_block"])
             return events_ms(lambda: ops.trace_paths(plan, pk, dt, M, check=False))
-        cfg = tuner().best(("trace block", *shape, M), lambda: [{"trace_block": b} for b in TRACE_BLOCKS], t_trace)
+        # (the segment tracer has one workgroup size: nothing to choose there)
+        blocks = TRACE_BLOCKS if _lib.lib().vct_plan_uses_trace_block(plan.handle, dt, M) else TRACE_BLOCKS[:1]
+        cfg = tuner().best(("trace block", *shape, M), lambda: [{"trace_block": b} for b in blocks], t_trace)
         plan.set_option(_lib.OPT_TRACE_BLOCK, cfg["trace_block"])
         chosen.update(cfg)
     if "adjoint" in what:

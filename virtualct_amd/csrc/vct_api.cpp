@@ -441,6 +441,11 @@ vct_status vct_plan_set_option(vct_plan* p, int option, int value)
     }
 }
 
+int vct_plan_uses_trace_block(const vct_plan* p, int dens_type, int M)
+{
+    return p && M >= 1 && M <= 8 && trace_uses_block(make_trace_args(p), dens_type, M) ? 1 : 0;
+}
+
 vct_status vct_plan_destroy(vct_plan* p)
 {
     if (!p) return VCT_OK;

@@ -193,6 +193,7 @@ struct vct_plan {
 namespace vct {
 // kernels launchers (implemented in the .hip files)
 vct_status launch_trace(const TraceArgs& a, int dens_type, int M, bool adjoint, hipStream_t s);
+bool trace_uses_block(const TraceArgs& a, int dens_type, int M);  // false: k_trace_seg, which has its own
 size_t trace_redo_words(int V, int W);  // 64-bit words of TraceArgs::redo
 vct_status launch_spectral(const SpectralArgs& a, hipStream_t s);
 vct_status launch_stats_init(uint32_t* stats, int S, hipStream_t s);

@@ -1740,6 +1740,11 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
     return VCT_OK;
 }
 
+bool trace_uses_block(const TraceArgs& a, int dens_type, int M)
+{
+    return !seg_grid(a, (dens_type == VCT_DENS_U16 ? 4 : 8) * ((M + 1) / 2));
+}
+
 size_t trace_redo_words(int V, int W)
 {
     return (size_t)((V + kSegViews - 1) / kSegViews) * (size_t)((W + kSegCh - 1) / kSegCh);
