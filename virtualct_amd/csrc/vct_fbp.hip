@@ -451,9 +451,13 @@ __device__ __forceinline__ void bp_multi_tile(const BackprojArgs& a, int S, int 
         } else {
 #pragma unroll
             for (int k = 0; k < K; k++) {
-                const float* p = fl[k] + row;
-                t0[k] = p[col];
-                t1[k] = p[col + 1];
+                // (one pointer: col + 1 as a 32-bit index may wrap, and the pair
+                // would be two loads, each of which spreads over as many lines
+                // where pixels are wider than channels: 256^2 x 800 views, 13
+                // sinograms, 379 us with one load, 599 with two)
+                const float* p = fl[k] + row + col;
+                t0[k] = p[0];
+                t1[k] = p[1];
             }
         }
     };
