@@ -320,7 +320,8 @@ vct_status vct_backproject(vct_plan* plan, const float* d_fltd, int n_sino, floa
 /* The same images bit for bit with a workspace of
  * vct_backproject_workspace_bytes(plan, n_sino) bytes (0: none is used), in
  * which several sinograms are interleaved in slices, at most 48 at a time, so
- * that a lane reads its sinograms' taps in 16-byte loads.  The size grows with
+ * that a lane reads its sinograms' taps in 16-byte loads (small calls go
+ * without).  The size grows with
  * n_sino and depends on no option, so a workspace for n_sino serves every
  * smaller call too.  d_work NULL: vct_backproject. */
 size_t vct_backproject_workspace_bytes(const vct_plan* plan, int n_sino);

@@ -466,7 +466,7 @@ def test_backprojection_workspace_serves_smaller_calls(gpu):
     import torch
     from virtualct_amd import _lib
     ops = _ops()
-    N, pix, V = 512, 0.1, 8
+    N, pix, V = 512, 0.1, 64
     plan = ops.Plan(_geom(N, pix, V))
     size = lambda n: int(_lib.lib().vct_backproject_workspace_bytes(plan.handle, n))
     sizes = []

@@ -194,9 +194,9 @@ def split(tmp_path_factory):
     src.write_text('#include "vct_split.h"\n'
                    'extern "C" void adjoint_split(int t, int v, int w, int a, int* o)\n'
                    '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n'
-                   'extern "C" int il_slots(int N, int cap, int S)\n'
-                   '{ int K = vct::bp_interleave_width(N, false, cap, S); return K ? vct::bp_interleave_slots(S, K) : 0; }\n'
-                   'extern "C" int il_bound(int S) { return vct::bp_interleave_bound(S); }\n')
+                   'extern "C" void il_split(int N, int v, int e, int cap, int S, int* o)\n'
+                   '{ auto s = vct::bp_interleave(N, v, e != 0, cap, S); o[0] = s.width; o[1] = s.per; }\n'
+                   'extern "C" int il_bound(int N, int v, int S) { return vct::bp_interleave_bound(N, v, S); }\n')
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "virtualct_amd", "csrc"),
                     str(src), "-o", str(lib)], check=True, capture_output=True)
     return C.CDLL(str(lib))
@@ -230,11 +230,24 @@ def test_adjoint_chunks_are_even_and_bounded(split):
 def test_interleave_bound_covers_every_smaller_call(split):
     """The workspace of several interleaved sinograms, sized for a count, serves
     every smaller count at every image size and option (50 sinograms at 512^2
-    use 40 slots, 48 use 48), and stays within one pass."""
-    bounds = [split.il_bound(n) for n in range(0, 60)]
-    assert bounds[:3] == [0, 0, 2] and bounds == sorted(bounds) and bounds[-1] == bounds[48] == 48
-    assert split.il_slots(512, 0, 50) == 40 and split.il_slots(512, 0, 48) == 48
+    use 40 slots, 48 use 48), and stays within one pass; small calls and small
+    images in several passes take no interleaving."""
+    out = (C.c_int * 2)()
+
+    def of(N, views, cap, S, exact=0):
+        split.il_split(N, views, exact, cap, S, out)
+        return out[0], out[1]
+    assert of(512, 800, 0, 50) == (10, 40) and of(512, 800, 0, 48) == (12, 48) and of(200, 360, 0, 50) == (10, 40)
+    assert of(64, 80, 0, 2)[0] == 2 and of(512, 50, 0, 4)[0] == 4 and of(128, 160, 0, 48)[0] == 6
+    assert of(16, 2, 0, 12)[0] == of(128, 40, 0, 4)[0] == of(128, 800, 0, 50)[0] == of(512, 800, 0, 12, 1)[0] == 0
+    counts = (*range(1, 100), 150, 65535)
     for N in (2, 64, 97, 128, 200, 300, 512, 8192):
-        for cap in (0, *range(2, 17)):
-            for n in (*range(1, 100), 65535):
-                assert split.il_slots(N, cap, n) <= bounds[min(n, 59)], (N, cap, n)
+        for views in (1, 40, 64, 800):
+            bounds = [split.il_bound(N, views, n) for n in counts]
+            assert bounds == sorted(bounds) and bounds[0] == 0 and bounds[-1] in (0, 48)
+            for cap in (0, *range(2, 17)):
+                for n, bound in zip(counts, bounds):
+                    K, per = of(N, views, cap, n)
+                    if K:
+                        assert K % 2 == 0 and K <= 12 and per % K == 0 and K <= per <= 48
+                        assert -(-min(n, per) // K) * K <= bound, (N, views, cap, n)

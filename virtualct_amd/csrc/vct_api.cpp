@@ -805,7 +805,8 @@ vct_status vct_backproject(vct_plan* p, const float* d_fltd, int n_sino, float* 
 size_t vct_backproject_workspace_bytes(const vct_plan* p, int n_sino)
 {
     if (!p || n_sino < 1) return 0;
-    return (size_t)bp_interleave_bound(std::min(n_sino, kIlPass)) * p->g.n_views * p->g.n_channels * sizeof(float);
+    return (size_t)bp_interleave_bound(p->g.recon_size, p->g.n_views, n_sino) * p->g.n_views * p->g.n_channels *
+           sizeof(float);
 }
 
 vct_status vct_backproject_ws(vct_plan* p, const float* d_fltd, int n_sino, float* d_img, void* d_work, void* stream)
@@ -814,13 +815,13 @@ vct_status vct_backproject_ws(vct_plan* p, const float* d_fltd, int n_sino, floa
     if (!p || !d_fltd || !d_img) return set_error(VCT_ERR_ARG, "NULL argument");
     if (n_sino < 1 || n_sino > 65535) return set_error(VCT_ERR_ARG, "n_sino %d invalid", n_sino);
     hipStream_t s = pick_stream(p, stream);
-    const int K = d_work ? bp_interleave_width(p->g.recon_size, p->exact_bp != 0, p->bp_max_k, n_sino) : 0;
-    if (K == 0) return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, s);
+    const Interleave il = bp_interleave(p->g.recon_size, p->g.n_views, p->exact_bp != 0, p->bp_max_k, n_sino);
+    const int K = il.width;
+    if (!d_work || K == 0) return launch_backproject(make_bp_args(p, d_fltd, d_img), n_sino, s);
     const int VW = p->g.n_views * p->g.n_channels;
     const size_t NN = (size_t)p->g.recon_size * p->g.recon_size;
-    const int pass = bp_interleave_pass(K);
-    for (int i = 0; i < n_sino; i += pass) {
-        const int n = std::min(n_sino - i, pass);
+    for (int i = 0; i < n_sino; i += il.per) {
+        const int n = std::min(n_sino - i, il.per);
         VCT_CHECK(launch_interleave_sinos(d_fltd + (size_t)i * VW, n, VW, K, (float*)d_work, s));
         VCT_CHECK(launch_backproject_il(make_bp_args(p, (const float*)d_work, d_img + i * NN), n, K, s));
     }

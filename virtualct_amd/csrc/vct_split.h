@@ -39,37 +39,55 @@ inline AdjointSplit adjoint_split(int ntiles, int views, int channels, int asked
 
 constexpr int kIlWidth = 12;  // widest slice
 constexpr int kIlPass = 48;   // most sinograms that one pass interleaves (bounds the workspace)
+constexpr long long kIlLanes = 1 << 17;  // lanes of a pass that fill the chip
 
-// Width of the interleaved slices that S sinograms of N^2 pixels take, 0 for
-// none (a single sinogram, the exact option).  The fewest slices of at most
-// kIlWidth (max_k: VCT_OPT_BP_SINOS_PER_LANE), but enough that the launch has
-// kIlLanes lanes, and then the narrowest width that holds an even share.
-// Measured (us, one launch, 800 views): 16 sinograms at 512^2 as 3 x 6, 2 x 8,
-// 12 + 4 and 1 x 16 867, 889, 1103 and 1235; 12 at 300^2 as 2 x 6, 12 and 3 x 4
-// 291, 319 and 363; 12 at 200^2 x 360 views as 3 x 4, 2 x 6, 12 and 6 x 2 104,
-// 114, 117 and 148.
-inline int bp_interleave_width(int N, bool exact, int max_k, int S)
+struct Interleave {
+    int width, per;  // sinograms per slice and per pass; width 0: not interleaved
+};
+
+// A call of so little work that the interleaving launch costs as much as it
+// saves: few views, whose chain of adds is short, on few pixels (us of the call,
+// plain and interleaved: 16^2 x 2 views 7 and 14, 32^2 x 40 11 and 14, 128^2 x 40
+// with 4 and 13 sinograms 11 and 14, 18 and 15; 64^2 x 80 19 and 20, x 800 170 to 248
+// and 144 to 170).
+inline bool bp_interleave_small(int N, int views, int S)
 {
-    constexpr long long kIlLanes = 1 << 17;
-    if (S < 2 || exact) return 0;
+    return views < 64 && (long long)N * N * views * S < 1 << 25;
+}
+
+// How S sinograms of N^2 pixels are interleaved: the fewest slices of at most
+// kIlWidth (max_k: VCT_OPT_BP_SINOS_PER_LANE), but enough that the launch has
+// kIlLanes lanes, and then the narrowest width that holds an even share, in
+// passes of as many whole slices as kIlPass holds.  Images so small that a whole
+// pass has fewer lanes run better in one plain launch than in several (50
+// sinograms, plain and interleaved: 128^2 x 160 views 79 and 132 us; 200^2 x 360
+// 404 and 369).  Measured (us, one launch, 800 views): 16 sinograms at 512^2 as
+// 3 x 6, 2 x 8, 12 + 4 and 1 x 16 867, 889, 1103 and 1235; 12 at 300^2 as 2 x 6,
+// 12 and 3 x 4 291, 319 and 363; 12 at 200^2 x 360 views as 3 x 4, 2 x 6, 12 and
+// 6 x 2 104, 114, 117 and 148.
+inline Interleave bp_interleave(int N, int views, bool exact, int max_k, int S)
+{
+    if (S < 2 || exact || bp_interleave_small(N, views, S)) return {0, S};
     const long long px = (long long)N * N;
     const int cap = max_k >= 2 && max_k < kIlWidth ? max_k / 2 * 2 : kIlWidth;
     const int slices = std::max((S + cap - 1) / cap, (int)std::min<long long>((S + 1) / 2, (kIlLanes + px - 1) / px));
-    return ((S + slices - 1) / slices + 1) / 2 * 2;
+    const int K = ((S + slices - 1) / slices + 1) / 2 * 2, per = kIlPass / K * K;
+    if (S > per && kIlPass / K * px < kIlLanes) return {0, S};
+    return {K, per};
 }
 
-// Sinograms per pass of slices of K, and the slots that S of them take.
-inline int bp_interleave_pass(int K) { return kIlPass / K * K; }
-inline int bp_interleave_slots(int S, int K) { return std::min((S + K - 1) / K * K, bp_interleave_pass(K)); }
+// Slots that n sinograms of one pass take in slices of K.
+inline int bp_interleave_slots(int n, int K) { return (n + K - 1) / K * K; }
 
 // Slots that serve up to S sinograms at any width that such a call can take,
 // whatever the options: it grows with S, so a workspace sized for the largest
 // call serves the others.
-inline int bp_interleave_bound(int S)
+inline int bp_interleave_bound(int N, int views, int S)
 {
+    if (S < 2 || bp_interleave_small(N, views, S)) return 0;
     int slots = 0;
     for (int K = 2; K <= std::min(kIlWidth, (S + 1) / 2 * 2); K += 2)
-        if (S >= 2) slots = std::max(slots, bp_interleave_slots(S, K));
+        slots = std::max(slots, bp_interleave_slots(std::min(S, kIlPass / K * K), K));
     return slots;
 }
 

@@ -291,7 +291,7 @@ def backproject(plan: Plan, fltd: torch.Tensor):
     fltd = _sinograms(plan, fltd, "filtered sinogram")
     S = fltd.shape[0]
     img = torch.empty((S, plan.N, plan.N), dtype=torch.float32, device=fltd.device)
-    need = int(_lib.lib().vct_backproject_workspace_bytes(plan.handle, S))
+    need = int(_lib.lib().vct_backproject_workspace_bytes(plan.handle, S)) if S > 1 else 0
     work = torch.empty(need, dtype=torch.uint8, device=fltd.device) if need else None
     call("vct_backproject_ws", plan.handle, _ptr(fltd), S, _ptr(img), _ptr(work) if need else None,
          _stream(plan.device))
