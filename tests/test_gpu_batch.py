@@ -615,3 +615,23 @@ def test_grouped_spectral_and_backprojection_equal_per_group_calls(gpu):
         batch.backproject_groups(list(zip(plans, fls, imgs)), k)
         for p, f, im in zip(plans, fls, imgs):
             assert torch.equal(im, ops.backproject(p, f)), (p.N, k)
+
+
+@pytest.mark.parametrize("V,B,S,NE,M", [(2, 1, 7, 40, 6), (8, 37, 7, 17, 8), (3, 150, 2, 33, 3), (81, 1, 5, 120, 1)])
+def test_batch_spectral_shared_spectra_equal_single_calls(gpu, V, B, S, NE, M):
+    """Few rays: the spectra of a phantom are shared by several workgroups (all
+    of them, an uneven part), each summed as in a call of one phantom, so the
+    values and the statistics are the same bits."""
+    import torch
+    ops, batch, _ = _mods()
+    from virtualct_amd import default_geometry
+    plan = ops.plan_for(default_geometry(recon_size=64, pixel_cm=0.7, n_views=V))
+    g = torch.Generator(device=gpu).manual_seed(V + B)
+    L = torch.rand((V * 609, B, 8), generator=g, device=gpu) * 10
+    L[..., M:] = 0
+    att = torch.rand((S, M, NE), generator=g, device=gpu) * 0.2
+    pdf = torch.rand((S, NE), generator=g, device=gpu) / NE
+    raw, stats = batch.batch_spectral(plan, batch.to_planes(L), M, att, pdf)
+    for b in {0, B // 2, B - 1}:
+        r1, s1, _ = ops.spectral_sum(plan, L[:, b].contiguous().view(V, 609, 8), M, att, pdf)
+        assert torch.equal(raw[b], r1) and torch.equal(stats[b], s1)

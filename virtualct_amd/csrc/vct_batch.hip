@@ -51,6 +51,7 @@
 #include "vct_internal.h"
 #include "vct_march.h"
 #include "vct_spectral.h"
+#include "vct_split.h"
 
 // Two-stage form of one direction (see above).
 struct vct_blocked {
@@ -618,9 +619,10 @@ __device__ __forceinline__ void spec_slot(const BatchSpecArgs& a, int z, const f
     b = z - a.pref[g];
 }
 
-// Forward mode: raw and per-(phantom, spectrum) max/min, all spectra of phantom
-// blockIdx.z, one after the other, in one block: the ray's path integrals are
-// loaded once, and the table of one spectrum at a time is in LDS (spec_sum).
+// Forward mode: raw and per-(phantom, spectrum) max/min, the spectra of phantom
+// blockIdx.z, one after the other, in one block (every gridDim.y-th of them,
+// spectral_parts): the ray's path integrals are loaded once, and the table of
+// one spectrum at a time is in LDS (spec_sum).
 // Rays per workgroup: each workgroup adds its max and min of each (phantom,
 // spectrum) to that pair's statistics words with one atomic each, which
 // serialise per address, so workgroups are large.
@@ -647,7 +649,7 @@ __global__ __launch_bounds__(kSpecAllBlock) void k_batch_spectral(BatchSpecArgs 
     SpecRays<M> L;
     L.load([&](int t, int m) { return ray0 + t < traced ? Lrows[slot_index(ray0 + t, B, b, m)] : 0.f; });
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int s = 0; s < S; s++) {
+    for (int s = blockIdx.y; s < S; s += gridDim.y) {
         const SpecTable<M> tab =
             SpecTable<M>::fill(lds, last, a.att + (size_t)s * M * NE, a.pdf + (size_t)s * NE, NE);
         float I = spec_sum<M>(tab, L);
@@ -2262,7 +2264,8 @@ static vct_status check_spec(vct_plan* p, const float* L, int B, int M, const fl
 
 static void launch_batch_spectral(const BatchSpecArgs& a, int M, int B, hipStream_t s)
 {
-    const dim3 grid((a.rays + kSpecAllBlock - 1) / kSpecAllBlock, 1, B), blk(kSpecAllBlock);
+    const int gx = (a.rays + kSpecAllBlock - 1) / kSpecAllBlock;
+    const dim3 grid(gx, spectral_parts(gx, B, a.S), B), blk(kSpecAllBlock);
     switch (M) {
 #define VCT_SPEC_CASE(MM)                                                                                            \
     case MM:                                                                                                         \
