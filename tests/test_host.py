@@ -194,6 +194,9 @@ def split(tmp_path_factory):
     src.write_text('#include "vct_split.h"\n'
                    'extern "C" void adjoint_split(int t, int v, int w, int a, int* o)\n'
                    '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n'
+                   'extern "C" int adjoint_lanes(int M, int n, int v, int c, int w, double t)\n'
+                   '{ return vct::adjoint_lanes(M, n, {v, c}, w, t); }\n'
+                   'extern "C" int spectral_parts(int r, int p, int s) { return vct::spectral_parts(r, p, s); }\n'
                    'extern "C" void il_split(int N, int v, int e, int cap, int S, int* o)\n'
                    '{ auto s = vct::bp_interleave(N, v, e != 0, cap, S); o[0] = s.width; o[1] = s.per; }\n'
                    'extern "C" int il_bound(int N, int v, int S) { return vct::bp_interleave_bound(N, v, S); }\n')
@@ -251,3 +254,18 @@ def test_interleave_bound_covers_every_smaller_call(split):
                     if K:
                         assert K % 2 == 0 and K <= 12 and per % K == 0 and K <= per <= 48
                         assert -(-min(n, per) // K) * K <= bound, (N, views, cap, n)
+
+
+def test_small_launches_are_split_by_their_work(split):
+    """The tile adjoint takes 256 lanes only where its rays leave half of 512
+    without one, the LDS holds three workgroups and the chip is full; a
+    phantom's spectra are shared only as far as the launch needs workgroups."""
+    def lanes(M, ntiles, views, chunks, channels, tile):
+        return split.adjoint_lanes(M, ntiles, views, chunks, channels, C.c_double(tile))
+    assert [lanes(M, 16, 1, 80, 609, 140.0) for M in range(1, 9)] == [256] * 6 + [512] * 2
+    assert lanes(6, 144, 52, 14, 609, 46.0) == lanes(1, 16, 2, 80, 609, 140.0) == 512
+    assert lanes(1, 1, 1, 4, 22, 140.0) == lanes(1, 16, 1, 80, 609, float("inf")) == 512
+    assert lanes(1, 600, 8, 1, 22, 1e9) == 256 and lanes(6, 600, 4, 1, 609, float("nan")) == 512
+    assert split.spectral_parts(5, 1, 64) == 64 and split.spectral_parts(476, 3, 2) == 1
+    assert split.spectral_parts(48, 1, 64) == 11 and split.spectral_parts(1, 65535, 64) == 1
+    assert split.spectral_parts(476, 1, 2) == 2 and split.spectral_parts(512, 1, 64) == 1

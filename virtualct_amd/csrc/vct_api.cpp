@@ -93,6 +93,7 @@ TraceArgs make_trace_args(const vct_plan* p)
     a.invD = 1.0 / g.pixel_cm;
     a.rmax = g.recon_size * 0.5 * 1.0;
     a.sid = g.sid_cm;
+    a.ch_cm = std::fabs(g.sid_cm * g.max_alpha / p->half);
     // The r >= rmax test of the reference (M/reprojection_TOMO.cpp:150-155)
     // compares a radius in cm with N/2 and only fires when a segment midpoint
     // can lie farther than N/2 cm from the centre.

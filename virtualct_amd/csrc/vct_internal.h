@@ -64,6 +64,7 @@ struct TraceArgs {
     double invD;          // 1/D (fast path for the voxel index, with exact fallback)
     double rmax;          // N*0.5 (reference :37)
     double sid;           // source to isocentre
+    double ch_cm;         // channel pitch at the isocentre
     double out_scale;     // factor applied to the accumulated sums (1/1000 for u16, then /xfactor)
 };
 

@@ -405,7 +405,7 @@ struct SinkRot {
 // form serves workgroups whose weights are not all finite, so NaN and
 // infinity reach the gradient as with float sums.
 constexpr int kAdjTile = 32;
-constexpr int kAdjBlock = 512;
+constexpr int kAdjBlock = 512;  // most lanes of a workgroup (adjoint_lanes)
 
 template <int M, bool FIXED>
 struct SinkTile {
@@ -1343,9 +1343,10 @@ __global__ __launch_bounds__(kAdjBlock, 4) void k_trace_adj_tile(TraceArgs a, in
     __syncthreads();
     const float* dens = reinterpret_cast<const float*>(a.dens);
     const double unscale = ldexp(1.0, -S);
-    // (eight lanes per voxel, so that a wave's adds cover whole lines of grad)
-    for (int i = threadIdx.x; i < TS * TS * 8; i += blockDim.x) {
-        const int m = i & 7, lx = (i >> 3) % TS, ly = (i >> 3) / TS;
+    // (a lane per material of a voxel, so that a wave's adds cover whole lines of grad)
+    constexpr int MP = M > 4 ? 8 : M > 2 ? 4 : M;
+    for (int i = threadIdx.x; i < TS * TS * MP; i += blockDim.x) {
+        const int m = i % MP, lx = i / MP % TS, ly = i / MP / TS;
         const int x = x0 + lx, y = y0 + ly;
         if (m >= M || x >= a.N || y >= a.N) continue;
         const size_t v = (size_t)y * a.N + x;
@@ -1723,7 +1724,8 @@ static vct_status launch_trace_m(const TraceArgs& a, int dens_type, bool adjoint
             const int ntx = (a.N + kAdjTile - 1) / kAdjTile, ntiles = ntx * ntx;
             const AdjointSplit sp = adjoint_split(ntiles, a.VT, a.W, a.adj_views);
             const int per_xcd = (ntiles * sp.chunks + 7) / 8;
-            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(kAdjBlock), 0, s, a, ntx, ntiles, sp.views,
+            const int lanes = adjoint_lanes(M, ntiles, sp, a.W, std::min(a.N, kAdjTile) * a.D / a.ch_cm);
+            hipLaunchKernelGGL((k_trace_adj_tile<M>), dim3(per_xcd * 8), dim3(lanes), 0, s, a, ntx, ntiles, sp.views,
                                per_xcd, seg_planes(a) ? 1 : 0);
         }
     } else if (!a.exact && a.n_rays <= INT_MAX / 8) {
