@@ -469,3 +469,32 @@ def test_lone_ray_segments_equal_exact_march(gpu, N, V, M, f32, orbit):
     assert ce.sum() > 0
     np.testing.assert_array_equal(c, ce)
     assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9)
+
+
+@pytest.mark.parametrize("V,M,f32", [(12, 6, False), (80, 8, True), (80, 1, False), (200, 8, False), (14, 2, True),
+                                      (50, 6, False), (162, 6, True), (5, 8, False), (15, 6, True), (61, 3, False)])
+def test_segment_workgroup_sizes_equal_exact_march(gpu, V, M, f32):
+    """Workgroups of 16, 32 and 64 orbits (few to many views) of 4, 2 and 1
+    rays, with last tiles that are not full and a channel whose ray passes
+    through the isocentre along the grid lines, which is left to the second
+    kernel in some views: the counters of the exact-division march and its path
+    integrals within two float roundings."""
+    from virtualct_amd import _lib, default_geometry
+    ops = _ops()
+    N, W = 130, 334
+    geom = default_geometry(recon_size=N, pixel_cm=49.3 / N, n_views=V, n_channels=W, iso_channel=W / 2.0)
+    rng = np.random.default_rng(V + M)
+    d = rng.uniform(0.0, 2.0, (M, N, N)).astype(np.float32) if f32 else \
+        rng.integers(0, 2000, (M, N, N)).astype(np.int16)
+    out = []
+    for exact in (0, 1):
+        plan = ops.Plan(geom)
+        plan.set_option(_lib.OPT_EXACT_TRACE, exact)
+        pk, dt = ops.pack_densities(plan, _t(d, gpu))
+        L, cnt = ops.trace_paths(plan, pk, dt, M, counts=True)
+        out.append((L.cpu().numpy(), cnt.cpu().numpy()))
+        plan.close()
+    (L, c), (Le, ce) = out
+    assert ce[:, W // 2].max() > 0
+    np.testing.assert_array_equal(c, ce)
+    assert np.all(np.abs(L - Le) <= 2.0 ** -22 * np.abs(Le) + 1e-9) and not np.any(L[..., M:])

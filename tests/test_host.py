@@ -194,6 +194,7 @@ def split(tmp_path_factory):
     src.write_text('#include "vct_split.h"\n'
                    'extern "C" void adjoint_split(int t, int v, int w, int a, int* o)\n'
                    '{ auto s = vct::adjoint_split(t, v, w, a); o[0] = s.views; o[1] = s.chunks; }\n'
+                   'extern "C" int seg_shift(int n, int b, int t) { return vct::seg_shift(n, b, t); }\n'
                    'extern "C" int adjoint_lanes(int M, int n, int v, int c, int w, double t)\n'
                    '{ return vct::adjoint_lanes(M, n, {v, c}, w, t); }\n'
                    'extern "C" int spectral_parts(int r, int p, int s) { return vct::spectral_parts(r, p, s); }\n'
@@ -259,7 +260,11 @@ def test_interleave_bound_covers_every_smaller_call(split):
 def test_small_launches_are_split_by_their_work(split):
     """The tile adjoint takes 256 lanes only where its rays leave half of 512
     without one, the LDS holds three workgroups and the chip is full; a
-    phantom's spectra are shared only as far as the launch needs workgroups."""
+    phantom's spectra are shared only as far as the launch needs workgroups; the
+    segment tracer takes fewer orbits per workgroup for few views."""
+    assert [split.seg_shift(1024, v // 4, 39) for v in (4, 40, 200, 400, 800)] == [4, 4, 5, 5, 6]
+    assert [split.seg_shift(64, v // 4, 39) for v in (4, 40, 80)] == [5, 5, 6] and split.seg_shift(2, 65536, 512) == 6
+    assert all(4 <= split.seg_shift(n, b, t) <= 6 for n in (2, 8192) for b in (1, 65536) for t in (2, 512))
     def lanes(M, ntiles, views, chunks, channels, tile):
         return split.adjoint_lanes(M, ntiles, views, chunks, channels, C.c_double(tile))
     assert [lanes(M, 16, 1, 80, 609, 140.0) for M in range(1, 9)] == [256] * 6 + [512] * 2

@@ -6,6 +6,25 @@
 
 namespace vct {
 
+// ------------------------------------------------ segment tracer (vct_trace.hip)
+
+// log2 of the orbits of a workgroup: 6, or 5 or 4 where n, the workgroups of 64
+// orbits (16 channels of 4 base views), are too few to share the chip's L1s; the
+// more voxels a march passes, the more they are worth against the closer lanes
+// of 64.  The densities' type and count do not enter (calls of a plan share the
+// redo bits, whose layout this is).  us with 64, 32 and 16 orbits, u16, M = 6, 609
+// channels (n): 1024^2 x 40 views (117) 271, 168, 148; x 160 (390) 567, 469, 462; x
+// 240 (585) 763, 583, 686; x 480 (1170) 881, 913, 1344; 512^2 x 40 102, 63, 54; x 160
+// 154, 116, 112; x 200 (507) 191, 127, 133; x 480 218, 215, 276; 256^2 x 80 (195) 43, 39,
+// 41; x 200 58, 59, 69; 128^2 x 40 28, 23, 24; x 160 36, 38, 49; 64^2 x 40 21, 19, 21; x 80
+// 21, 23, 29.
+inline int seg_shift(int N, int base_views, int channel_tiles)
+{
+    const double n = (base_views + 3) / 4 * (double)channel_tiles;
+    if (n <= std::min(0.6 * N, 350.0)) return 4;
+    return n <= std::min(std::max(1.8 * N, 128.0), 1000.0) ? 5 : 6;
+}
+
 // ------------------------------------------------- tile adjoint (vct_trace.hip)
 
 constexpr int kAdjMaxViews = 256;  // views per workgroup (its tables in LDS)

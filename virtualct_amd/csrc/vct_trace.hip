@@ -735,14 +735,17 @@ __global__ __launch_bounds__(256) void k_trace_fwd_rot(TraceArgs a)
 // about the same place and its gathers fall into few cache lines: requests to
 // L2 bound the tracer before the instructions do (64 channels of one view per
 // wave drift apart by rows: 0.44 ms where 16 x 4 take 0.30; 8 x 8 and 32 x 2
-// 0.31 and 0.32; eight windows of eight orbits, the split before, 0.53).  The
-// windows' sums meet in LDS, one ray of the orbits after the other.
+// 0.31 and 0.32; eight windows of eight orbits, the split before, 0.53).  Few
+// views make too few such workgroups for the chip's L1s: they hold 32 or 16
+// orbits then, in 16 or 32 windows (seg_shift).  The windows' sums meet in LDS,
+// one ray of the orbits after the other.
 // 800 x 609, against k_trace_fwd_rot: u16 M = 6 512^2 0.53 -> 0.29 ms, M = 8
 // 0.62 -> 0.33; float M = 6 512^2 1.08 -> 0.48, 768^2 2.53 -> 0.95; one ray
 // per march (401 views) against k_trace_fwd 0.60 -> 0.28.  Orbits read the
 // plan's work copies; one ray per march reads the packed densities, so that
 // calls of such a plan (odd views or grid) on several streams stay apart: the
-// redo bits, which all calls share, depend on the geometry alone.
+// redo bits, which all calls share, and the orbits per workgroup, which lay them
+// out, depend on the geometry alone.
 constexpr int kSegWaves = 8;
 
 // Bytes per voxel of the tracer's work copies: the materials in use.
@@ -752,14 +755,14 @@ constexpr int seg_voxel()
     return DT == VCT_DENS_U16 ? 4 * ((M + 1) / 2) : 8 * ((M + 1) / 2);
 }
 
-// A workgroup's 64 orbits: kSegCh neighbouring channels of 64 / kSegCh
+// A workgroup's 16 V orbits (V = 4, 2 or 1): kSegCh neighbouring channels of V
 // neighbouring base views.
-constexpr int kSegCh = 16, kSegViews = 64 / kSegCh;
-__host__ __device__ __forceinline__ void seg_orbit(int block, int lane, int W, int& view, int& ch)
+constexpr int kSegCh = 16;
+__host__ __device__ __forceinline__ void seg_orbit(int block, int orbit, int V, int W, int& view, int& ch)
 {
     const int ct = (W + kSegCh - 1) / kSegCh, vt = block / ct;
-    view = vt * kSegViews + lane / kSegCh;
-    ch = (block - vt * ct) * kSegCh + lane % kSegCh;
+    view = vt * V + orbit / kSegCh;
+    ch = (block - vt * ct) * kSegCh + orbit % kSegCh;
 }
 
 template <int M, int DT, int R>
@@ -847,16 +850,17 @@ struct SegSums {
 };
 
 template <int M, int DT, int R>
-__global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
+__global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a, int sh)
 {
     using Sums = SegSums<M, DT, R>;
     constexpr int VB = Sums::VB;
-    __shared__ double part[kSegWaves][M][64];
+    __shared__ double part[64 * kSegWaves * M];  // [window][material][orbit]
     __shared__ int cnt[64], redo[64];
-    const int lane = threadIdx.x & 63, piece = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // 2^sh orbits (seg_shift), of which a lane marches one in one of the windows
+    const int pieces = 64 * kSegWaves >> sh, lane = threadIdx.x & ((1 << sh) - 1), piece = (int)threadIdx.x >> sh;
     const int Vq = (R == 1 ? a.VT : a.V / R);
     int view, ch;
-    seg_orbit(blockIdx.x, lane, a.W, view, ch);
+    seg_orbit(blockIdx.x, lane, (1 << sh) / kSegCh, a.W, view, ch);
     const bool valid = view < Vq && ch < a.W;
     if (piece == 0) {
         cnt[lane] = 0;
@@ -883,8 +887,8 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
         bad = !((fabs(ai) == Lb || trunc_safe(ai)) && fabs(af - ai) >= kMarchMargin &&
                 fabs(r.bf - r.bi) >= kMarchMargin && fabs(kBA) <= 1.0e6);
         // window of planes: this piece ends segments at planes k0 .. kstop
-        const int len = (march_step_estimate(a, r) + kSegWaves - 1) / kSegWaves;
-        const int k0 = max(piece * len, 1), k1 = piece == kSegWaves - 1 ? a.max_steps : (piece + 1) * len - 1;
+        const int len = (march_step_estimate(a, r) + pieces - 1) / pieces;
+        const int k0 = max(piece * len, 1), k1 = piece == pieces - 1 ? a.max_steps : (piece + 1) * len - 1;
         // last plane inside the square (exactly u_0 + fl(k D) <= Lb)
         int ka = (int)fmin(fmax((Lb - uain) / D, -1.0), 1.0e8);
         if (uain + (double)(ka + 1) * D <= Lb) ka++;
@@ -1077,44 +1081,51 @@ __global__ __launch_bounds__(64 * kSegWaves) void k_trace_seg(TraceArgs a)
         if (!bad && n) atomicAdd(&cnt[lane], n);
     }
     if (bad) redo[lane] = 1;
-    // the windows' sums, ray k of the 64 orbits at a time: wave w adds and
-    // writes slots w, w + kSegWaves, .. of every orbit
+    // the windows' sums, ray k of the orbits at a time: lane t adds and writes
+    // slot t >> sh of its orbit
     const bool xmaj = hit && r.xmajor;
 #pragma unroll
     for (int k = 0; k < R; k++) {
         __syncthreads();
 #pragma unroll
-        for (int m = 0; m < M; m++) part[piece][m][lane] = sums.sum(k, m);
+        for (int m = 0; m < M; m++) part[((piece * M + m) << sh) + lane] = sums.sum(k, m);
         __syncthreads();
         // slots 1 and 3 hold rays 3 and 1 when y is the base ray's major axis
         const int ray_k = (R == 4 && (k & 1) && !xmaj) ? 4 - k : k;
-        if (valid && !redo[lane]) {
-            const int ray = (view + ray_k * Vq) * a.W + ch;
-            float* dst = a.L + (size_t)ray * 8;
-            for (int m = piece; m < 8; m += kSegWaves) {
-                double t = 0.0;
-                if (m < M) {
+        if (valid && !redo[lane] && piece < 8) {
+            const int ray = (view + ray_k * Vq) * a.W + ch, m = piece;
+            double t = 0.0;
+            if (m < M) {
+                auto eight = [&](int w0) {
 #pragma unroll
-                    for (int w = 0; w < kSegWaves; w++) t += part[w][m][lane];
+                    for (int w = 0; w < kSegWaves; w++) t += part[(((w0 + w) * M + m) << sh) + lane];
+                };
+                // (not a loop: with one the compiler forms all rays' sums before it,
+                // in half as many registers again)
+                eight(0);
+                if (sh < 6) eight(8);
+                if (sh < 5) {
+                    eight(16);
+                    eight(24);
                 }
-                dst[m] = (float)(t * a.out_scale);
             }
+            a.L[(size_t)ray * 8 + m] = (float)(t * a.out_scale);
             if (piece == 0 && a.counts) a.counts[ray] = cnt[lane];
         }
     }
-    if (piece == 0) {
-        const unsigned long long m = __ballot(valid && redo[lane]);
-        if (lane == 0) a.redo[blockIdx.x] = m;
+    if (threadIdx.x < 64) {
+        const unsigned long long m = __ballot(piece == 0 && valid && redo[lane]);
+        if (threadIdx.x == 0) a.redo[blockIdx.x] = m;
     }
 }
 
-// The rays of the orbits that k_trace_seg left (bit l of redo[w]: lane l of
+// The rays of the orbits that k_trace_seg left (bit l of redo[w]: orbit l of
 // workgroup w), each by its own march in the 64 windows of a wave (a kernel of
 // its own, so that the general march's registers do not count against the
 // segment loop's).  One workgroup, a wave per ray of an orbit, per 64 words;
 // they are nearly always all zero.
 template <int M, int DT, int R>
-__global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words)
+__global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words, int sh)
 {
     constexpr int P = 64;
     using Sink = std::conditional_t<DT == VCT_DENS_U16, SinkU16<M>, SinkF32<M>>;
@@ -1127,7 +1138,7 @@ __global__ __launch_bounds__(64 * R) void k_trace_redo(TraceArgs a, int words)
         unsigned long long m = __shfl(mine, w);
         while (m) {
             int v0, ch;
-            seg_orbit(w0 + w, __ffsll((long long)m) - 1, a.W, v0, ch);
+            seg_orbit(w0 + w, __ffsll((long long)m) - 1, (1 << sh) / kSegCh, a.W, v0, ch);
             m &= m - 1;
             const int view = v0 + (int)(threadIdx.x >> 6) * Vq, piece = lane;
             RayConst r;
@@ -1671,7 +1682,8 @@ static vct_status launch_trace_seg(const TraceArgs& a, hipStream_t s)
 {
     if (a.rot > 1) launch_pack_copies<DT == VCT_DENS_U16 ? 16 : 32, seg_voxel<M, DT>(), DT == VCT_DENS_F32>(a, s);
     const int base_views = a.rot > 1 ? a.V / a.rot : a.VT;
-    const dim3 grid((unsigned)(((base_views + kSegViews - 1) / kSegViews) * ((a.W + kSegCh - 1) / kSegCh)));
+    const int ct = (a.W + kSegCh - 1) / kSegCh, sh = seg_shift(a.N, base_views, ct), vt = (1 << sh) / kSegCh;
+    const dim3 grid((unsigned)((base_views + vt - 1) / vt * ct));
     const dim3 block(64 * kSegWaves);
     if (a.VT < a.V) {
         // an odd count's last view is not traced
@@ -1683,8 +1695,8 @@ static vct_status launch_trace_seg(const TraceArgs& a, hipStream_t s)
         const int words = (int)grid.x;
         const dim3 rgrid((unsigned)((words + 63) / 64));
 #define VCT_SEG(RR)                                                                  \
-    hipLaunchKernelGGL((k_trace_seg<M, DT, RR>), grid, block, 0, s, a);              \
-    hipLaunchKernelGGL((k_trace_redo<M, DT, RR>), rgrid, dim3(64 * RR), 0, s, a, words);
+    hipLaunchKernelGGL((k_trace_seg<M, DT, RR>), grid, block, 0, s, a, sh);          \
+    hipLaunchKernelGGL((k_trace_redo<M, DT, RR>), rgrid, dim3(64 * RR), 0, s, a, words, sh);
         if (a.rot == 4) { VCT_SEG(4) }
         else if (a.rot == 2) { VCT_SEG(2) }
         else { VCT_SEG(1) }
@@ -1749,7 +1761,7 @@ bool trace_uses_block(const TraceArgs& a, int dens_type, int M)
 
 size_t trace_redo_words(int V, int W)
 {
-    return (size_t)((V + kSegViews - 1) / kSegViews) * (size_t)((W + kSegCh - 1) / kSegCh);
+    return (size_t)V * (size_t)((W + kSegCh - 1) / kSegCh);
 }
 
 vct_status launch_trace(const TraceArgs& a, int dens_type, int M, bool adjoint, hipStream_t s)
