@@ -440,7 +440,7 @@ def main():
             "note": "algorithmic bytes = segments x 6 materials x 2 B (u16 densities) + V x W x 4 B; the "
                     "traffic is what the L2s fetch and write; the gathers are served by the caches, so the "
                     "algorithmic rate can exceed the HBM peak, and the kernel is bound by FP64 VALU issue "
-                    "(28 VALU instructions per ray-segment, 83% VALU busy)",
+                    "(29 VALU instructions per ray-segment, 83% VALU busy)",
         },
         "rooflines": [
             {"kernel": "k_trace_seg (tracer, quarter-turn orbits)", "bound": "hbm", "unit": "GB/s", "achieved": achieved,
@@ -454,7 +454,7 @@ def main():
              "per_launch": "P_mask x V x 8 B + N^2 x 4 B = %.3f GB" % (bp_bytes / 1e9),
              "note": "the taps come from the 1.95 MB filtered sinogram held in L2 (16.6 MB of traffic "
                      "past the L2s per launch), so the algorithmic rate can exceed the HBM peak; the "
-                     "kernel is bound by VALU issue (66% busy, 12 VALU instructions per masked "
+                     "kernel is bound by VALU issue (69% busy, 12 VALU instructions per masked "
                      "pixel-view) and its gathers"},
         ],
         "cpu_baseline": None,

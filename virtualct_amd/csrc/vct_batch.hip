@@ -68,7 +68,7 @@ struct vct_blocked {
 // that lane l of a wave reads entries 4 q .. 4 q + 3 of run l at slice_ptr +
 // 256 q + 4 l: a 16-byte load of lengths and an 8-byte load of LDS indices.
 //   forward: a block is a 64x64 image tile; an entry holds its voxel's index
-//     inside the tile (ly * 64 + lx) and the length; padding entries are
+//     inside the tile (ly * 67 + lx) and the length; padding entries are
 //     (kTilePadVoxel, 0.0f), which read zeroed LDS;
 //   adjoint: a block is (view block, part of a 64x64 image tile), whose LDS
 //     table holds, view after view, the rays of the view block that cross
@@ -1200,12 +1200,11 @@ __global__ __launch_bounds__(256) void k_weights_pm(const float* __restrict__ in
 // (round-robin dispatch) and takes phantom b of block xcd_tiles[xcd][k], so
 // the B workgroups of a block share one L2 for its entries.
 //   forward: the tile's M materials of phantom b go to LDS (64 rows of 64
-//     voxels x MP floats, rows padded by 2 floats so that voxels one row
-//     apart fall 2 banks apart);
+//     voxels x MP floats, rows 67 voxels apart: kTilePitch);
 //   adjoint: the M weights of phantom b of the block's rays go to LDS, slot
 //     after slot (MP floats each), slot 0 zero.
-// Each lane then sums one run of a slice in FP64, 8 entries in flight, and
-// writes its partial sums as stage-1 row run, phantom b.  The sums are those
+// Each lane then sums one run of a slice in FP64, three register sets of four
+// entries in turn, two of them in flight, and writes its partial sums as stage-1 row run, phantom b.  The sums are those
 // of k_gather over the same runs, term for term in the same order.
 // Bound by what passes between L2 and the CU: at 16 phantoms of 512^2, M = 6,
 // a copy without the LDS reads or without the sums takes the same 3.8 ms, one

@@ -23,6 +23,8 @@
 //   k_backproject_sym  one sinogram by orbits of the quarter turn: each
 //                  pixel-view geometry serves four pixels (views a multiple
 //                  of 4, N even; sums in another order).
+//   k_backproject_lone  one sinogram on other grids and view counts: orbits of
+//                  four, two or one pixels, FP64 sums.
 #include "vct_internal.h"
 
 #include <algorithm>

@@ -151,7 +151,7 @@ __device__ __forceinline__ double rsq_refined(double x)
 // expression.
 //
 // FP64 issue bounds both forms (about 55 vector instructions per pixel-view
-// here): 2.08 -> 0.47 ms at 512^2, 800 views.  Four waves share 64 pixels: each
+// here): 2.00 -> 0.44 ms at 512^2, 800 views.  Four waves share 64 pixels: each
 // computes kNpfChunk views of a round into LDS and the first adds them, views
 // ascending.  One pixel per lane with all its views took 0.50 ms (every
 // workgroup is resident from the start, and those on the mask's edge leave

@@ -26,7 +26,7 @@
 //                split over eight lanes by step windows, for the grids that
 //                k_trace_seg does not take (seg_grid).
 //   k_trace_adj_tile  the adjoint by image tiles: windowed marches of the
-//                rays that cross a tile, w_m * length summed in LDS in 64-bit
+//                rays that cross a tile, w_m * length summed in LDS in
 //                fixed point, one float atomic per voxel at the end.
 #include "vct_internal.h"
 #include "vct_march.h"
@@ -1209,7 +1209,8 @@ static bool seg_planes(const TraceArgs& a)
 // bound it.  Two workgroups of 512 lanes per CU within 128 registers instead
 // of three of 256 lanes with 135: 380^2 x 722 views, M = 6, 1.38 -> 1.16 ms,
 // M = 8 1.87 -> 1.28; the addend by one fused multiply-add 1.53 -> 1.38; the
-// segment loop 1.91 -> 1.53; larger tiles (40) 1.11, but 0.14 instead of 0.12
+// segment loop 1.91 -> 1.53; workgroups with few rays take 256 lanes
+// (adjoint_lanes); larger tiles (40) 1.11, but 0.14 instead of 0.12
 // at 64^2.
 template <int M>
 __device__ __forceinline__ void adj_weights(const TraceArgs& a, int ray, float (&w)[M])

@@ -58,7 +58,7 @@ class Plan:
         # voxel-major system matrix, built on first use (8 bytes per segment
         # in each direction, 4.5 GB at 512^2 / 800 x 609; ~70 ms), atomic-free
         # and deterministic, 1.5 ms per call at 512^2; "atomic" re-traces the
-        # rays tile by tile (2.7 ms per call, no memory beyond the gradient).
+        # rays tile by tile (1.6 ms per call, no memory beyond the gradient).
         self.adjoint_mode = "sysmat"
         self._sysmat = None
 
