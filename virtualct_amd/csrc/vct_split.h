@@ -62,7 +62,8 @@ inline AdjointSplit adjoint_split(int ntiles, int views, int channels, int asked
 // more and idle lanes for less.  M = 1 and 6, 512 and 256 lanes: 128^2 x 80
 // views on 51.2 cm (178 rays) 172 and 190 us, 133 and 165; 512^2 x 40 views of 300
 // channels 192 and 206, 140 and 170; 256^2 x 100 views (340 rays) 154 and 172, 144
-// and 184; 101^2 x 80 (220 rays) 108 and 130, 91 and 138; M = 8 at 128^2 203 and 214; 8^2 x 4 views of 22 channels, M = 6, 17 and 19.
+// and 184; 101^2 x 80 (220 rays) 108 and 130, 91 and 138; M = 8 at 128^2 203 and 214; 8^2
+// x 4 views of 22 channels, M = 6, 17 and 19.
 inline int adjoint_lanes(int M, int ntiles, AdjointSplit sp, int channels, double tile_channels)
 {
     const bool few = sp.views * std::min((double)channels, 1.27 * tile_channels) <= 256.0 - 8.0 * M;
